@@ -41,6 +41,7 @@ struct fx_mesh {
     int* err = nullptr;      // [code, dir, x, y, z, stage]
     int integrator = FX_RK2;
     int riemann = FX_RIEMANN_HLLC;   // hydro meshes
+    int split = 1;           // hydro: stage workgroups per block
     int ct_split = 1;        // MHD CT workgroups per block
     // MHD meshes whose flux kernel fits the chip in one round (at most 2
     // workgroups per CU): stream and events on which the ghost-layer face
@@ -131,6 +132,16 @@ int read_error_word(fx_mesh* m)
     return FX_OK;
 }
 
+// compute units of the current device
+hipError_t cu_count(int& ncu)
+{
+    int dev_id = 0;
+    hipError_t e = hipGetDevice(&dev_id);
+    if (e == hipSuccess)
+        e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev_id);
+    return e;
+}
+
 // host global [nh][X][Y][Z] <-> device padded, per (var, x) plane
 int copy_cells(fx_mesh* m, double* dev, const double* host_in, double* host_out, int nh)
 {
@@ -200,6 +211,7 @@ int run_stage(fx_mesh* m, int stage, const double* dt_ptr, double dt)
         a.dt = dt;
         a.cfl_part = stage == 2 ? m->dev + 8 : nullptr;
         a.riemann = m->riemann;
+        a.split = m->split;
         hipEvent_t e0 = nullptr, e1 = nullptr;
         if (m->timing) {
             FX_HIP(hipEventCreate(&e0));
@@ -317,23 +329,23 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
         if (e == hipSuccess) e = hipMalloc(&m->fdat, 9 * m->cell_bytes);
         if (e == hipSuccess) e = hipMalloc(&m->zring, zring_doubles(m->g) * sizeof(double));
     }
+    m->nblocks = m->g.nbx * m->g.nby * m->g.nbz;
+    int ncu = 0;
+    if (e == hipSuccess) e = cu_count(ncu);
+    if (e == hipSuccess && !desc->mhd) m->split = hydro_split(m->nblocks, ncu);
     if (e == hipSuccess && desc->mhd) {
-        int dev_id = 0, ncu = 0;
-        e = hipGetDevice(&dev_id);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev_id);
-        if (e == hipSuccess) m->ct_split = mhd_ct_split(m->g, ncu);
-        const int64_t nb = (int64_t)m->g.nbx * m->g.nby * m->g.nbz;
-        if (e == hipSuccess && nb <= 2 * (int64_t)ncu) {
+        m->ct_split = mhd_ct_split(m->g, ncu);
+        const int64_t nb = m->nblocks;
+        if (nb <= 2 * (int64_t)ncu) {
             e = create_side_stream(m);
             m->side_on = e == hipSuccess;
         }
     }
     // dev[0..7] scalars, then the CFL partials: one per workgroup of the
     // reduction, or the maxima a stage 2 records
-    m->nblocks = m->g.nbx * m->g.nby * m->g.nbz;
-    m->cfl_nparts = m->nblocks * (desc->mhd ? m->ct_split : 1);
+    m->cfl_nparts = m->nblocks * (desc->mhd ? m->ct_split : m->split);
     // room for the partials of the largest CT split fx_mesh_set_mhd_schedule allows
-    const size_t npart = (size_t)std::max(CALC_DT_WGS, m->nblocks * (desc->mhd ? 4 : 1));
+    const size_t npart = (size_t)std::max(CALC_DT_WGS, m->nblocks * (desc->mhd ? 4 : m->split));
     if (e == hipSuccess) e = hipMalloc(&m->dev, (8 + npart) * sizeof(double));
     if (e == hipSuccess) e = hipMemset(m->dev, 0, 8 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&m->err, 8 * sizeof(int));
@@ -485,9 +497,8 @@ int fx_mesh_set_mhd_schedule(fx_mesh* m, int ct_split, int side_stream)
         return fail(FX_EINVAL, "side_stream must be -1 (automatic), 0 or 1");
     FX_HIP(hipStreamSynchronize(m->stream));
     if (m->side) FX_HIP(hipStreamSynchronize(m->side));
-    int dev_id = 0, ncu = 0;
-    FX_HIP(hipGetDevice(&dev_id));
-    FX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev_id));
+    int ncu = 0;
+    FX_HIP(cu_count(ncu));
     m->ct_split = ct_split != 0 ? ct_split : mhd_ct_split(m->g, ncu);
     m->cfl_nparts = m->nblocks * m->ct_split;
     m->cfl_ready = false;   // recorded per CT workgroup of the old split
@@ -753,9 +764,11 @@ struct fx_ensemble {
     EnsBlock* d_blocks[2] = {nullptr, nullptr};
     int* d_queues = nullptr;
     double* dev = nullptr;               // 4 doubles per instance
-    double* partial = nullptr;           // per-block CFL maxima of the per-instance schedule
+    double* partial = nullptr;           // CFL maxima of the per-instance schedule, per workgroup
     std::vector<int> part_off;           // first partial of each instance
+    std::vector<int> split1;             // stage workgroups per block of each instance alone
     int nblocks = 0;
+    int split = 1;                       // stage workgroups per block of the batched launches
     // the CFL maxima of the current states are recorded (dev[2] of every
     // instance in the batched schedule, `partial` in the per-instance one)
     bool cfl_ready = false;
@@ -784,6 +797,9 @@ void ens_drop_graph(fx_ensemble* e)
 
 int ens_nblocks(const Geom& g) { return g.nbx * g.nby * g.nbz; }
 
+// CFL partials of instance i in the per-instance schedule
+int ens_nparts(const fx_ensemble* e, int i) { return ens_nblocks(e->geoms[i]) * e->split1[i]; }
+
 // CFL maxima of the current states, read from the cells, where the step
 // expects them (a stage 2 records them for the step after it)
 int ens_enqueue_cfl(fx_ensemble* e)
@@ -792,7 +808,7 @@ int ens_enqueue_cfl(fx_ensemble* e)
     if (e->mode == 0) {
         for (int i = 0; i < e->n; ++i) {
             const EnsInst& I = e->host_inst[i];
-            FX_HIP(launch_dt_reduce(I.g, I.W[0], e->partial + e->part_off[i], ens_nblocks(I.g), s));
+            FX_HIP(launch_dt_reduce(I.g, I.W[0], e->partial + e->part_off[i], ens_nparts(e, i), s));
         }
         return FX_OK;
     }
@@ -808,7 +824,7 @@ int ens_enqueue_step(fx_ensemble* e, double cfl, double factor)
         for (int i = 0; i < e->n; ++i) {
             const EnsInst& I = e->host_inst[i];
             double* part = e->partial + e->part_off[i];
-            FX_HIP(launch_dt_final(part, ens_nblocks(I.g), cfl, I.dev + 0, I.dev + 1, factor, 1.0, s));
+            FX_HIP(launch_dt_final(part, ens_nparts(e, i), cfl, I.dev + 0, I.dev + 1, factor, 1.0, s));
             for (int st = 1; st <= 2; ++st) {
                 double* Win = st == 1 ? I.W[0] : I.W[1];
                 HydroStageArgs a;
@@ -819,6 +835,7 @@ int ens_enqueue_step(fx_ensemble* e, double cfl, double factor)
                 a.dt_ptr = I.dev;
                 a.dt = 0.0;
                 a.cfl_part = st == 2 ? part : nullptr;
+                a.split = e->split1[i];
                 FX_HIP(launch_hydro_stage(a, st, s));
             }
         }
@@ -828,8 +845,8 @@ int ens_enqueue_step(fx_ensemble* e, double cfl, double factor)
     FX_HIP(launch_ens_dt_finalize(e->d_inst, e->n, cfl, factor, s));
     for (int st = 1; st <= 2; ++st) {
         if (st == 2) FX_HIP(launch_ens_dt_clear(e->d_inst, e->n, s));
-        FX_HIP(launch_ens_stage(e->d_inst, tbl, e->nblocks, st, e->persistent_wgs, e->xcd, e->xcd,
-                                e->d_queues, s));
+        FX_HIP(launch_ens_stage(e->d_inst, tbl, e->nblocks, st, e->split, e->persistent_wgs, e->xcd,
+                                e->xcd, e->d_queues, s));
     }
     return FX_OK;
 }
@@ -898,11 +915,15 @@ int fx_ensemble_create(int n, const fx_mesh_desc* descs, fx_ensemble** out)
                 for (int bz = 0; bz < g.nbz; ++bz) e->order[0].push_back({i, bx, by, bz});
     }
     e->nblocks = (int)e->order[0].size();
-    for (int i = 0, acc = 0; i < n; ++i) {
-        e->part_off.push_back(acc);
-        acc += ens_nblocks(e->geoms[i]);
+    int ncu = 0, nparts = 0;
+    if (err == hipSuccess) err = cu_count(ncu);
+    e->split = hydro_split(e->nblocks, ncu);
+    for (int i = 0; i < (int)e->geoms.size(); ++i) {
+        e->split1.push_back(hydro_split(ens_nblocks(e->geoms[i]), ncu));
+        e->part_off.push_back(nparts);
+        nparts += ens_nparts(e, i);
     }
-    if (err == hipSuccess) err = hipMalloc(&e->partial, (size_t)std::max(1, e->nblocks) * sizeof(double));
+    if (err == hipSuccess) err = hipMalloc(&e->partial, (size_t)std::max(1, nparts) * sizeof(double));
     // interleaved table: instances dealt round robin block by block, so that
     // every part of the table mixes all instances
     {
@@ -1069,10 +1090,8 @@ int fx_ensemble_autotune(fx_ensemble* e, double cfl, double dt_factor, int reps,
                          double* best_ms)
 {
     if (e == nullptr || reps <= 0) return fail(FX_EINVAL, "bad autotune arguments");
-    int dev_id = 0;
-    FX_HIP(hipGetDevice(&dev_id));
     int ncu = 0;
-    FX_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev_id));
+    FX_HIP(cu_count(ncu));
     const int cand[][4] = {
         {1, 0, 1, 0}, {1, 0, 0, 0}, {1, 0, 1, 1},
         {1, ncu, 1, 0}, {1, 2 * ncu, 1, 0}, {1, 2 * ncu, 0, 1},

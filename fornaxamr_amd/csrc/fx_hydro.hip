@@ -161,7 +161,9 @@ struct HydroLds {
 // limiter, or HLLE (same face states and wave-speed bounds, no contact)
 enum { RS_HLLC = 0, RS_HLLE = 1 };
 
-// One RK2 stage of block (bx, by, bz) of the mesh described by g.  Called by
+// One RK2 stage of np x-planes (np <= 16, from x0) of the 16 x 16 cell columns
+// at (y0, z0) of the mesh described by g: a whole block, or one part of a block
+// whose planes are split over several workgroups.  Called by
 // the single-mesh kernel and by the batched ensemble kernels.  Stage 2 returns
 // the largest CFL denominator of the cells this thread wrote (the next step's
 // time-step reduction, taken while the new state is in registers); stage 1
@@ -171,8 +173,8 @@ template <int STAGE, int RS = RS_HLLC>
 __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
                                             const double* __restrict__ Win,
                                             const double* __restrict__ W0,
-                                            double* __restrict__ Wout, double dt, int bx, int by,
-                                            int bz)
+                                            double* __restrict__ Wout, double dt, int x0, int np,
+                                            int y0, int z0)
 {
     auto& pl = L.pl;
     auto& v1p = L.v1p;
@@ -187,7 +189,6 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
     const int lane = t & 63;
     const int wave = t >> 6;
     const int wv = __builtin_amdgcn_readfirstlane(wave);   // the same, as a scalar
-    const int x0 = bx * BS, y0 = by * BS, z0 = bz * BS;
     const int64_t vs = g.vstride;
     const double gm1 = g.gamma - 1.0;
     const double gam = g.gamma;
@@ -219,7 +220,7 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
     const int64_t col_own = cell_off(g, 0, y0 + j, z0 + k);
     const int64_t col_halo = cell_off(g, 0, hym, hzm);
 
-    // active planes (p in [0, BS)): the update and W^n
+    // active planes (p in [0, np)): the update and W^n
     auto own_at = [&](int p) { return col_own + (int64_t)(x0 + p) * g.sx; };
     // plane p of the stencil, mapped; fx receives its x flip bit
     auto plane_x = [&](int p, int& fx) {
@@ -305,7 +306,7 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
         for (int q = 0; q < 6; ++q) w0n[q] = W0[q * vs + own_at(0)];
     }
 
-    for (int i = 0; i < BS; ++i) {
+    for (int i = 0; i < np; ++i) {
         const int A = i & 1;
         const int B = A ^ 1;
         // the wave with one pass more than the others before the next barrier
@@ -517,7 +518,7 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
 #pragma unroll
             for (int v = 0; v < 6; ++v) fd[v] = fs[v] / vol;
         }
-        if (i < BS - 1) store_plane(pl[A], pf, oidx, hidx, has_halo);
+        if (i < np - 1) store_plane(pl[A], pf, oidx, hidx, has_halo);
 
         // ---- per-cell RK2 update -------------------------------------------
         {
@@ -548,8 +549,8 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
 
 #pragma unroll
         for (int q = 0; q < 6; ++q) Fx[q] = Fxn[q];
-        if (i + 3 <= BS + 1) load_at(i + 3, pf);
-        if (STAGE == 2 && i + 1 < BS) {
+        if (i + 3 <= np + 1) load_at(i + 3, pf);
+        if (STAGE == 2 && i + 1 < np) {
 #pragma unroll
             for (int q = 0; q < 6; ++q) w0n[q] = W0[q * vs + own_at(i + 1)];
         }
@@ -562,28 +563,39 @@ __global__ void __launch_bounds__(NT, 2) hydro_stage_kernel(HydroStageArgs a)
 {
     __shared__ HydroLds L;
     const Geom& g = a.g;
-    const int b = block_of_workgroup(blockIdx.x, gridDim.x);
+    // workgroup -> (part, block): a block's x-planes may be split over several
+    // workgroups (hydro_split), each with its own prologue; the face between
+    // two parts is formed by both, from the same cells
+    const int wg = block_of_workgroup(blockIdx.x, gridDim.x);
+    const int np = BS / a.split;
+    const int part = wg % a.split;
+    const int b = wg / a.split;
     const int bz = b % g.nbz;
     const int by = (b / g.nbz) % g.nby;
     const int bx = b / (g.nbz * g.nby);
     const double dt = a.dt_ptr ? *a.dt_ptr : a.dt;
-    const double d = hydro_block<STAGE, RS>(L, g, a.Win, a.W0, a.Wout, dt, bx, by, bz);
+    const double d = hydro_block<STAGE, RS>(L, g, a.Win, a.W0, a.Wout, dt, bx * BS + part * np, np,
+                                            by * BS, bz * BS);
     if (STAGE == 2 && a.cfl_part != nullptr) {
         const double m = workgroup_max(d, L.v1p[0]);
-        if (threadIdx.x == 0) a.cfl_part[b] = m;
+        if (threadIdx.x == 0) a.cfl_part[wg] = m;
     }
 }
 
-// One table entry of a batched stage: block (bx, by, bz) of instance `inst`.
+// Entry b of a batched stage over a table of (instance, block) entries whose
+// x-planes are split over `split` workgroups: part b % split of the block
+// (bx, by, bz) of instance `inst` at table index b / split.
 template <int STAGE>
 __device__ __forceinline__ void ens_entry(HydroLds& L, const EnsInst* __restrict__ inst,
-                                          const EnsBlock* __restrict__ blocks, int b)
+                                          const EnsBlock* __restrict__ blocks, int split, int b)
 {
-    const EnsBlock e = blocks[b];
+    const EnsBlock e = blocks[b / split];
+    const int np = BS / split;
     const EnsInst& I = inst[e.inst];
     const double dt = I.dev[0];
     const double d = hydro_block<STAGE>(L, I.g, I.W[STAGE == 1 ? 0 : 1], I.W[0],
-                                        I.W[STAGE == 1 ? 1 : 0], dt, e.bx, e.by, e.bz);
+                                        I.W[STAGE == 1 ? 1 : 0], dt,
+                                        e.bx * BS + (b % split) * np, np, e.by * BS, e.bz * BS);
     if (STAGE == 2) {
         // dev[2] holds the bits of the instance's largest denominator
         // (non-negative doubles order as their bit patterns); the step clears
@@ -603,11 +615,12 @@ __device__ __forceinline__ void ens_entry(HydroLds& L, const EnsInst* __restrict
 // entry; XCD_REMAP gives every XCD a contiguous run of the table.
 template <int STAGE, int XCD_REMAP>
 __global__ void __launch_bounds__(NT, 2) ens_stage_kernel(const EnsInst* __restrict__ inst,
-                                                      const EnsBlock* __restrict__ blocks)
+                                                      const EnsBlock* __restrict__ blocks,
+                                                      int split)
 {
     __shared__ HydroLds L;
     const int b = XCD_REMAP ? block_of_workgroup(blockIdx.x, gridDim.x) : (int)blockIdx.x;
-    ens_entry<STAGE>(L, inst, blocks, b);
+    ens_entry<STAGE>(L, inst, blocks, split, b);
 }
 
 // Persistent batched stage: a fixed number of workgroups pull table entries
@@ -618,23 +631,24 @@ __global__ void __launch_bounds__(NT, 2) ens_stage_kernel(const EnsInst* __restr
 template <int STAGE, int XCD_QUEUES>
 __global__ void __launch_bounds__(NT, 2) ens_stage_persistent_kernel(const EnsInst* __restrict__ inst,
                                                                  const EnsBlock* __restrict__ blocks,
-                                                                 int nblocks, int* queues)
+                                                                 int split, int nentries,
+                                                                 int* queues)
 {
     __shared__ HydroLds L;
     __shared__ int s_b;
     const int nq = XCD_QUEUES ? 8 : 1;
-    const int per = (nblocks + nq - 1) / nq;
+    const int per = (nentries + nq - 1) / nq;
     for (int r = 0; r < nq; ++r) {
         const int q = XCD_QUEUES ? (int)((blockIdx.x + r) & 7) : 0;
         const int lo = q * per;
-        const int hi = min(nblocks, lo + per);
+        const int hi = min(nentries, lo + per);
         for (;;) {
             if (threadIdx.x == 0) s_b = lo + atomicAdd(&queues[q], 1);
             __syncthreads();
             const int b = __builtin_amdgcn_readfirstlane(s_b);
             __syncthreads();
             if (b >= hi) break;
-            ens_entry<STAGE>(L, inst, blocks, b);
+            ens_entry<STAGE>(L, inst, blocks, split, b);
             // The entry's stage-2 epilogue raises the CFL maximum from wave 1
             // (thread 64), never from the fetching lane; this barrier also
             // keeps the two apart.  (An earlier build had both on thread 0 and
@@ -653,44 +667,81 @@ __global__ void queue_reset_kernel(int* q)
 
 }  // namespace
 
+// A workgroup of np planes costs a prologue (five plane loads, an extra x-face)
+// and np plane steps; 2 ncu workgroups run at once.  In plane steps: one round
+// costs 1.5 + np (0.8 of it where every CU holds one workgroup at most), and in
+// longer runs, where prologues overlap other workgroups' planes, each full
+// round 0.85 + np and the last one 0.68 or 0.97 of that.  The constants are
+// from stage times of all five splits on 13 meshes of 8 to 1728 blocks (256
+// CUs); the split of the least estimate was the fastest measured one, or within
+// 1 % of it, on each.  Stage 1 unsplit -> split: 8 blocks 109 -> 17 us
+// (split 16), 64 blocks 113 -> 28 us (8), 125 blocks 114 -> 48 us (4), 216
+// blocks 113 -> 78 us (2), 343 blocks 148 -> 122 us (4); 512 blocks stay whole
+// (141 us, split 2: 146), as do 4096.
+int hydro_split(int64_t nblocks, int ncu)
+{
+    int best = 1;
+    double least = 0.0;
+    for (int split = 1; split <= BS; split *= 2) {
+        const int64_t w = nblocks * split, slots = 2 * (int64_t)ncu;
+        if (slots <= 0 || (split > 1 && w > 8 * slots)) break;
+        const double np = BS / split;
+        double t;
+        if (w <= slots) {
+            t = (w <= ncu ? 0.8 : 1.0) * (1.5 + np);
+        } else {
+            const int64_t rest = w % slots;
+            t = ((double)(w / slots) + (rest == 0 ? 0.0 : (rest <= ncu ? 0.68 : 0.97))) * (0.85 + np);
+        }
+        if (split == 1 || t < least) {
+            best = split;
+            least = t;
+        }
+    }
+    return best;
+}
+
 hipError_t launch_hydro_stage(const HydroStageArgs& a, int stage, hipStream_t stream)
 {
-    const int nblocks = a.g.nbx * a.g.nby * a.g.nbz;
+    if (a.split < 1 || a.split > BS || BS % a.split != 0) return hipErrorInvalidValue;
+    const int nwg = a.g.nbx * a.g.nby * a.g.nbz * a.split;
     const bool hlle = a.riemann == FX_RIEMANN_HLLE;
     if (stage == 1) {
-        if (hlle) hipLaunchKernelGGL((hydro_stage_kernel<1, RS_HLLE>), dim3(nblocks), dim3(NT), 0, stream, a);
-        else hipLaunchKernelGGL((hydro_stage_kernel<1, RS_HLLC>), dim3(nblocks), dim3(NT), 0, stream, a);
+        if (hlle) hipLaunchKernelGGL((hydro_stage_kernel<1, RS_HLLE>), dim3(nwg), dim3(NT), 0, stream, a);
+        else hipLaunchKernelGGL((hydro_stage_kernel<1, RS_HLLC>), dim3(nwg), dim3(NT), 0, stream, a);
     } else {
-        if (hlle) hipLaunchKernelGGL((hydro_stage_kernel<2, RS_HLLE>), dim3(nblocks), dim3(NT), 0, stream, a);
-        else hipLaunchKernelGGL((hydro_stage_kernel<2, RS_HLLC>), dim3(nblocks), dim3(NT), 0, stream, a);
+        if (hlle) hipLaunchKernelGGL((hydro_stage_kernel<2, RS_HLLE>), dim3(nwg), dim3(NT), 0, stream, a);
+        else hipLaunchKernelGGL((hydro_stage_kernel<2, RS_HLLC>), dim3(nwg), dim3(NT), 0, stream, a);
     }
     return hipGetLastError();
 }
 
 
 hipError_t launch_ens_stage(const EnsInst* inst, const EnsBlock* blocks, int nblocks, int stage,
-                            int persistent_wgs, int xcd_remap, int xcd_queues, int* queues,
-                            hipStream_t s)
+                            int split, int persistent_wgs, int xcd_remap, int xcd_queues,
+                            int* queues, hipStream_t s)
 {
     if (nblocks <= 0) return hipSuccess;
+    if (split < 1 || split > BS || BS % split != 0) return hipErrorInvalidValue;
+    const int n = nblocks * split;
     if (persistent_wgs <= 0) {
         if (stage == 1) {
-            if (xcd_remap) hipLaunchKernelGGL((ens_stage_kernel<1, 1>), dim3(nblocks), dim3(NT), 0, s, inst, blocks);
-            else hipLaunchKernelGGL((ens_stage_kernel<1, 0>), dim3(nblocks), dim3(NT), 0, s, inst, blocks);
+            if (xcd_remap) hipLaunchKernelGGL((ens_stage_kernel<1, 1>), dim3(n), dim3(NT), 0, s, inst, blocks, split);
+            else hipLaunchKernelGGL((ens_stage_kernel<1, 0>), dim3(n), dim3(NT), 0, s, inst, blocks, split);
         } else {
-            if (xcd_remap) hipLaunchKernelGGL((ens_stage_kernel<2, 1>), dim3(nblocks), dim3(NT), 0, s, inst, blocks);
-            else hipLaunchKernelGGL((ens_stage_kernel<2, 0>), dim3(nblocks), dim3(NT), 0, s, inst, blocks);
+            if (xcd_remap) hipLaunchKernelGGL((ens_stage_kernel<2, 1>), dim3(n), dim3(NT), 0, s, inst, blocks, split);
+            else hipLaunchKernelGGL((ens_stage_kernel<2, 0>), dim3(n), dim3(NT), 0, s, inst, blocks, split);
         }
         return hipGetLastError();
     }
     hipLaunchKernelGGL(queue_reset_kernel, dim3(1), dim3(64), 0, s, queues);
     const dim3 grid(persistent_wgs);
     if (stage == 1) {
-        if (xcd_queues) hipLaunchKernelGGL((ens_stage_persistent_kernel<1, 1>), grid, dim3(NT), 0, s, inst, blocks, nblocks, queues);
-        else hipLaunchKernelGGL((ens_stage_persistent_kernel<1, 0>), grid, dim3(NT), 0, s, inst, blocks, nblocks, queues);
+        if (xcd_queues) hipLaunchKernelGGL((ens_stage_persistent_kernel<1, 1>), grid, dim3(NT), 0, s, inst, blocks, split, n, queues);
+        else hipLaunchKernelGGL((ens_stage_persistent_kernel<1, 0>), grid, dim3(NT), 0, s, inst, blocks, split, n, queues);
     } else {
-        if (xcd_queues) hipLaunchKernelGGL((ens_stage_persistent_kernel<2, 1>), grid, dim3(NT), 0, s, inst, blocks, nblocks, queues);
-        else hipLaunchKernelGGL((ens_stage_persistent_kernel<2, 0>), grid, dim3(NT), 0, s, inst, blocks, nblocks, queues);
+        if (xcd_queues) hipLaunchKernelGGL((ens_stage_persistent_kernel<2, 1>), grid, dim3(NT), 0, s, inst, blocks, split, n, queues);
+        else hipLaunchKernelGGL((ens_stage_persistent_kernel<2, 0>), grid, dim3(NT), 0, s, inst, blocks, split, n, queues);
     }
     return hipGetLastError();
 }

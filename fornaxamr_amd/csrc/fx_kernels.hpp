@@ -18,8 +18,9 @@ struct HydroStageArgs {
     double* Wout;           // stage output (may alias W0 for stage 2)
     const double* dt_ptr;   // device dt, or null to use dt
     double dt;
-    // stage 2: cfl_part[b] = largest CFL denominator of block b's output
-    // (b = (bx * nby + by) * nbz + bz); null: not recorded
+    int split = 1;          // workgroups per block (1, 2, 4, 8 or 16), each 16 / split x-planes
+    // stage 2: cfl_part[w] = largest CFL denominator of the cells workgroup w
+    // wrote (nblocks * split entries); null: not recorded
     double* cfl_part = nullptr;
     int riemann = 0;        // FX_RIEMANN_HLLC or FX_RIEMANN_HLLE
 };
@@ -67,9 +68,11 @@ hipError_t launch_ens_dt_finalize(const EnsInst* inst, int ninst, double cfl, do
 // persistent_wgs == 0: one workgroup per table entry (XCD remap if xcd_remap);
 // otherwise that many persistent workgroups pull table entries from `queues`
 // (8 counters, one per XCD chunk when xcd_queues, else only the first).
+// Every block's x-planes are split over `split` entries, adjacent in the table's
+// order.
 hipError_t launch_ens_stage(const EnsInst* inst, const EnsBlock* blocks, int nblocks, int stage,
-                            int persistent_wgs, int xcd_remap, int xcd_queues, int* queues,
-                            hipStream_t s);
+                            int split, int persistent_wgs, int xcd_remap, int xcd_queues,
+                            int* queues, hipStream_t s);
 
 // Compact copies of the MHD ghost planes z = -1 and z = nz (the 9 cell
 // variables over x, y in [-2, n + 2)), which the ghost-layer face kernel reads
@@ -93,6 +96,8 @@ hipError_t launch_boundary_fill(const Geom& g, double* W, const double* bf, doub
                                 hipStream_t s);
 
 hipError_t launch_hydro_stage(const HydroStageArgs& a, int stage, hipStream_t s);
+// workgroups per block of a stage over nblocks blocks on a GPU of ncu CUs
+int hydro_split(int64_t nblocks, int ncu);
 
 // side (optional, with the events fork/join): a second stream on which the
 // ghost-layer face kernel runs beside the flux kernel; the CT kernel waits

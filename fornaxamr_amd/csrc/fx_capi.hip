@@ -41,7 +41,7 @@ struct fx_mesh {
     int* err = nullptr;      // [code, dir, x, y, z, stage]
     int integrator = FX_RK2;
     int riemann = FX_RIEMANN_HLLC;   // hydro meshes
-    int split = 1;           // hydro: stage workgroups per block
+    int split = 1;           // workgroups per block of the hydro stage / the MHD flux kernel
     int ct_split = 1;        // MHD CT workgroups per block
     // MHD meshes whose flux kernel fits the chip in one round (at most 2
     // workgroups per CU): stream and events on which the ghost-layer face
@@ -245,6 +245,7 @@ int run_stage(fx_mesh* m, int stage, const double* dt_ptr, double dt)
     a.err = m->err;
     a.dt_ptr = dt_ptr;
     a.dt = dt;
+    a.flux_split = m->split;
     a.ct_split = m->ct_split;
     a.cfl_part = stage == 2 ? m->dev + 8 : nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -332,9 +333,9 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
     m->nblocks = m->g.nbx * m->g.nby * m->g.nbz;
     int ncu = 0;
     if (e == hipSuccess) e = cu_count(ncu);
-    if (e == hipSuccess && !desc->mhd) m->split = hydro_split(m->nblocks, ncu);
+    if (e == hipSuccess) m->split = stage_split(m->nblocks, ncu);
     if (e == hipSuccess && desc->mhd) {
-        m->ct_split = mhd_ct_split(m->g, ncu);
+        m->ct_split = mhd_ct_split(m->nblocks, ncu);
         const int64_t nb = m->nblocks;
         if (nb <= 2 * (int64_t)ncu) {
             e = create_side_stream(m);
@@ -344,8 +345,10 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
     // dev[0..7] scalars, then the CFL partials: one per workgroup of the
     // reduction, or the maxima a stage 2 records
     m->cfl_nparts = m->nblocks * (desc->mhd ? m->ct_split : m->split);
-    // room for the partials of the largest CT split fx_mesh_set_mhd_schedule allows
-    const size_t npart = (size_t)std::max(CALC_DT_WGS, m->nblocks * (desc->mhd ? 4 : m->split));
+    // room for the partials of the largest CT split: the automatic one, or 4 by
+    // fx_mesh_set_mhd_schedule
+    const size_t npart = std::max<size_t>(
+        CALC_DT_WGS, (size_t)m->nblocks * (desc->mhd ? std::max(4, m->ct_split) : m->split));
     if (e == hipSuccess) e = hipMalloc(&m->dev, (8 + npart) * sizeof(double));
     if (e == hipSuccess) e = hipMemset(m->dev, 0, 8 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc(&m->err, 8 * sizeof(int));
@@ -499,7 +502,7 @@ int fx_mesh_set_mhd_schedule(fx_mesh* m, int ct_split, int side_stream)
     if (m->side) FX_HIP(hipStreamSynchronize(m->side));
     int ncu = 0;
     FX_HIP(cu_count(ncu));
-    m->ct_split = ct_split != 0 ? ct_split : mhd_ct_split(m->g, ncu);
+    m->ct_split = ct_split != 0 ? ct_split : mhd_ct_split(m->nblocks, ncu);
     m->cfl_nparts = m->nblocks * m->ct_split;
     m->cfl_ready = false;   // recorded per CT workgroup of the old split
     bool on = side_stream == 1 || (side_stream == -1 && m->nblocks <= 2 * ncu);
@@ -917,9 +920,9 @@ int fx_ensemble_create(int n, const fx_mesh_desc* descs, fx_ensemble** out)
     e->nblocks = (int)e->order[0].size();
     int ncu = 0, nparts = 0;
     if (err == hipSuccess) err = cu_count(ncu);
-    e->split = hydro_split(e->nblocks, ncu);
+    e->split = stage_split(e->nblocks, ncu);
     for (int i = 0; i < (int)e->geoms.size(); ++i) {
-        e->split1.push_back(hydro_split(ens_nblocks(e->geoms[i]), ncu));
+        e->split1.push_back(stage_split(ens_nblocks(e->geoms[i]), ncu));
         e->part_off.push_back(nparts);
         nparts += ens_nparts(e, i);
     }

@@ -564,7 +564,7 @@ __global__ void __launch_bounds__(NT, 2) hydro_stage_kernel(HydroStageArgs a)
     __shared__ HydroLds L;
     const Geom& g = a.g;
     // workgroup -> (part, block): a block's x-planes may be split over several
-    // workgroups (hydro_split), each with its own prologue; the face between
+    // workgroups (stage_split), each with its own prologue; the face between
     // two parts is formed by both, from the same cells
     const int wg = block_of_workgroup(blockIdx.x, gridDim.x);
     const int np = BS / a.split;
@@ -667,18 +667,21 @@ __global__ void queue_reset_kernel(int* q)
 
 }  // namespace
 
-// A workgroup of np planes costs a prologue (five plane loads, an extra x-face)
-// and np plane steps; 2 ncu workgroups run at once.  In plane steps: one round
+// Shared with the MHD flux kernel, which marches the same way at the same two
+// workgroups per CU.  A workgroup of np planes costs a prologue (the stencil's
+// planes, an extra x-face) and np plane steps; 2 ncu workgroups run at once.  In plane steps: one round
 // costs 1.5 + np (0.8 of it where every CU holds one workgroup at most), and in
 // longer runs, where prologues overlap other workgroups' planes, each full
 // round 0.85 + np and the last one 0.68 or 0.97 of that.  The constants are
-// from stage times of all five splits on 13 meshes of 8 to 1728 blocks (256
-// CUs); the split of the least estimate was the fastest measured one, or within
-// 1 % of it, on each.  Stage 1 unsplit -> split: 8 blocks 109 -> 17 us
-// (split 16), 64 blocks 113 -> 28 us (8), 125 blocks 114 -> 48 us (4), 216
-// blocks 113 -> 78 us (2), 343 blocks 148 -> 122 us (4); 512 blocks stay whole
-// (141 us, split 2: 146), as do 4096.
-int hydro_split(int64_t nblocks, int ncu)
+// from hydro stage times of all five splits on 13 meshes of 8 to 1728 blocks
+// (256 CUs); the split of the least estimate was the fastest measured one, or
+// within 1 % (MHD steps: 2 %) of it, on each.  Hydro stage 1 unsplit -> split:
+// 8 blocks 109 -> 17 us (split 16), 64 blocks 113 -> 28 us (8), 125 blocks
+// 114 -> 48 us (4), 216 blocks 113 -> 78 us (2), 343 blocks 148 -> 122 us (4);
+// 512 blocks stay whole (141 us, split 2: 146), as do 4096.  MHD step by the
+// flux split alone: 8 blocks 597 -> 158 us (16), 64 blocks 616 -> 249 us (8),
+// 125 blocks 648 -> 354 us (4), 216 blocks 715 -> 553 us (2).
+int stage_split(int64_t nblocks, int ncu)
 {
     int best = 1;
     double least = 0.0;

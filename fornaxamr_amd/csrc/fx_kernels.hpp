@@ -38,7 +38,8 @@ struct MhdStageArgs {
     int* err;               // device error word: [code, dir, x, y, z]
     const double* dt_ptr;
     double dt;
-    int ct_split = 1;       // CT workgroups per block (1, 2 or 4), each BS / ct_split x-planes
+    int flux_split = 1;     // flux workgroups per block (1, 2, 4, 8 or 16), each BS / flux_split x-planes
+    int ct_split = 1;       // CT workgroups per block, likewise
     // stage 2: cfl_part[w] = largest CFL denominator of the cells CT workgroup
     // w wrote (nblocks * ct_split entries); null: not recorded
     double* cfl_part = nullptr;
@@ -96,8 +97,9 @@ hipError_t launch_boundary_fill(const Geom& g, double* W, const double* bf, doub
                                 hipStream_t s);
 
 hipError_t launch_hydro_stage(const HydroStageArgs& a, int stage, hipStream_t s);
-// workgroups per block of a stage over nblocks blocks on a GPU of ncu CUs
-int hydro_split(int64_t nblocks, int ncu);
+// workgroups per block of the hydro stage or the MHD flux kernel over nblocks
+// blocks on a GPU of ncu CUs
+int stage_split(int64_t nblocks, int ncu);
 
 // side (optional, with the events fork/join): a second stream on which the
 // ghost-layer face kernel runs beside the flux kernel; the CT kernel waits
@@ -105,8 +107,8 @@ int hydro_split(int64_t nblocks, int ncu);
 hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s,
                             hipStream_t side = nullptr, hipEvent_t fork = nullptr,
                             hipEvent_t join = nullptr);
-// CT workgroups per block: more on meshes with fewer blocks than CT slots
-int mhd_ct_split(const Geom& g, int ncu);
+// CT workgroups per block of a stage over nblocks blocks on a GPU of ncu CUs
+int mhd_ct_split(int64_t nblocks, int ncu);
 
 // cell-centred B of the active cells from the faces (prj_mhd_bf2bc)
 hipError_t launch_bf2bc(const Geom& g, double* W, const double* bf, hipStream_t s);

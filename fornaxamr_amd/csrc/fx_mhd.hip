@@ -154,11 +154,18 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a)
     const int j = t >> 4;
     const int k = t & 15;
     const int lane = t & 63;
-    const int b = block_of_workgroup(blockIdx.x, gridDim.x);
+    // workgroup -> (x-part, block): a block's x-planes may be split over
+    // flux_split workgroups, each marching np planes from x0 with its own
+    // prologue; the x-face between two parts is formed by both, from the same
+    // cells: identical values
+    const int wg = block_of_workgroup(blockIdx.x, gridDim.x);
+    const int np = BS / a.flux_split;
+    const int part = wg % a.flux_split;
+    const int b = wg / a.flux_split;
     const int bz = b % g.nbz;
     const int by = (b / g.nbz) % g.nby;
     const int bx = b / (g.nbz * g.nby);
-    const int x0 = bx * BS, y0 = by * BS, z0 = bz * BS;
+    const int x0 = bx * BS + part * np, y0 = by * BS, z0 = bz * BS;
     const int64_t vs = g.vstride;
     const double gm1 = g.gamma - 1.0;
     const double gam = g.gamma;
@@ -249,7 +256,7 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a)
     const double* bfy = a.bf_in + g.fvstride;
     const double* bfz = a.bf_in + 2 * g.fvstride;
 
-    for (int i = 0; i < BS; ++i) {
+    for (int i = 0; i < np; ++i) {
         const int A = i & 1;       // LDS slot of plane i, and its exchange buffers
         const int B = A ^ 1;       // plane i + 1
         // ---- y/z faces of plane i ------------------------------------------
@@ -313,7 +320,7 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a)
         // halo cell of plane i+2, loaded here so that its latency overlaps the
         // divergence and update below (it goes to LDS at the end of the plane)
         double hh[9];
-        if (has_halo && i < BS - 1) {
+        if (has_halo && i < np - 1) {
 #pragma unroll
             for (int q = 0; q < 9; ++q) hh[q] = a.Win[q * vs + halo_at(i + 2)];
         }
@@ -379,7 +386,7 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a)
 #pragma unroll
         for (int v = 0; v < 6; ++v) Fx[v] = Fxn[v];
         // ---- plane i+2 into the slot of plane i ----------------------------
-        if (i < BS - 1) {
+        if (i < np - 1) {
 #pragma unroll
             for (int q = 0; q < NQ; ++q) pl[A][q][oidx] = c2[q];
             if (has_halo) {
@@ -828,12 +835,15 @@ int64_t ghostface_count(const Geom& g)
 
 }  // namespace
 
-int mhd_ct_split(const Geom& g, int ncu)
+// CT workgroups per block: the most that the chip holds at once (4 per CU, by
+// its 36-38 KB of LDS each).  MHD steps by this split, us: 8 blocks 330 / 216 /
+// 158 / 129 / 115 for 1 / 2 / 4 / 8 / 16; 64 blocks 449 / 315 / 249 / 222 / 214;
+// 105 blocks 532 / 398 / 341 / 317 / 333 (840 workgroups at 8); 216 blocks 743 /
+// 617 / 554 / 576 / 615; 768 blocks 1672 / 1714 / 1699.
+int mhd_ct_split(int64_t nblocks, int ncu)
 {
-    // the CT kernel holds 4 workgroups per CU (36 KB LDS each)
-    const int64_t nblocks = (int64_t)g.nbx * g.nby * g.nbz;
     int split = 1;
-    while (split < 4 && nblocks * split * 2 <= 4 * (int64_t)ncu) split *= 2;
+    while (split < BS && nblocks * split * 2 <= 4 * (int64_t)ncu) split *= 2;
     return split;
 }
 
@@ -841,9 +851,10 @@ hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s, hip
                             hipEvent_t fork, hipEvent_t join)
 {
     const int nblocks = a.g.nbx * a.g.nby * a.g.nbz;
-    if (a.ct_split != 1 && a.ct_split != 2 && a.ct_split != 4) return hipErrorInvalidValue;
+    if (a.ct_split < 1 || a.ct_split > BS || BS % a.ct_split != 0) return hipErrorInvalidValue;
+    if (a.flux_split < 1 || a.flux_split > BS || BS % a.flux_split != 0) return hipErrorInvalidValue;
     if (side != nullptr && (fork == nullptr || join == nullptr)) return hipErrorInvalidValue;
-    const int nct = nblocks * a.ct_split;
+    const int nfl = nblocks * a.flux_split, nct = nblocks * a.ct_split;
     const int64_t ngf = ghostface_count(a.g);
     if (ngf >= ((int64_t)1 << 31)) return hipErrorInvalidValue;   // 32-bit decode
     // The ghost-layer faces and the flux kernel's faces are disjoint sets of
@@ -861,8 +872,8 @@ hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s, hip
     if (side != nullptr) {
         if (hipError_t e = hipEventRecord(join, side)) return e;
     }
-    if (stage == 1) hipLaunchKernelGGL(mhd_flux_kernel<1>, dim3(nblocks), dim3(NT), 0, s, a);
-    else hipLaunchKernelGGL(mhd_flux_kernel<2>, dim3(nblocks), dim3(NT), 0, s, a);
+    if (stage == 1) hipLaunchKernelGGL(mhd_flux_kernel<1>, dim3(nfl), dim3(NT), 0, s, a);
+    else hipLaunchKernelGGL(mhd_flux_kernel<2>, dim3(nfl), dim3(NT), 0, s, a);
     if (side != nullptr) {
         if (hipError_t e = hipStreamWaitEvent(s, join, 0)) return e;
     }

@@ -53,3 +53,24 @@ def test_ensemble_parts(gpu, edges, schedule):
         assert om.step(0.4) == dts[i]
         assert np.array_equal(e.get_prim(i), om.W0)
     e.close()
+
+
+@pytest.mark.parametrize("n,eta", [
+    ((32, 32, 16), 0.0),        # flux 16 parts, CT 16
+    ((64, 48, 80), 1.0e-3),     # 8, 16; blocks not a multiple of 8
+    ((96, 64, 80), 0.0),        # 4, 8
+    ((96, 96, 96), 0.0),        # 2, 4
+    ((112, 96, 112), 1.0e-3),   # 4, 2
+])
+def test_mhd_parts(gpu, n, eta):
+    from fornaxamr_amd.mesh import GpuMesh
+    pr = P.random_smooth(n=n, seed=sum(n), bc=(0,) * 6, mhd=True, eta=eta)
+    gm = GpuMesh.from_problem(pr)
+    om = O.OracleSim(pr.n, pr.xlim, pr.bc, pr.gamma, mhd=True, eta=eta, log_cr=True)
+    om.set_state(pr.W, pr.bf)
+    for _ in range(2):
+        assert gm.step(pr.cfl) == om.step(pr.cfl)
+        assert np.array_equal(gm.get_prim(0), om.W0)
+        for a, b in zip(gm.get_bf(0), om.bf0):
+            assert np.array_equal(a, b)
+    gm.close()

@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <mutex>
 #include <string>
 #include <algorithm>
 #include <vector>
@@ -21,6 +22,16 @@
 #include "fx_kernels.hpp"
 
 using namespace fx;
+
+// Device staging of the host transfers of one mesh or ensemble: allocated by the
+// first transfer, at most STAGING_BYTES (one row if that is longer), freed with
+// its owner.
+constexpr size_t STAGING_BYTES = (size_t)64 << 20;
+struct Staging {
+    std::mutex lock;         // held by a transfer to its end
+    double* buf = nullptr;
+    size_t cap = 0;          // bytes
+};
 
 struct fx_mesh {
     Geom g;
@@ -56,6 +67,7 @@ struct fx_mesh {
     double* saved_bf[2] = {nullptr, nullptr};   // and their face fields (MHD)
     hipStream_t stream = nullptr;
     size_t cell_bytes = 0;   // bytes of one padded variable
+    Staging staging;         // host transfers
     // optional event timing of the stage kernels (excluding the ghost fill)
     bool timing = false;
     struct Span { hipEvent_t a, b; int stage; };
@@ -142,47 +154,86 @@ hipError_t cu_count(int& ncu)
     return e;
 }
 
-// host global [nh][X][Y][Z] <-> device padded, per (var, x) plane
-int copy_cells(fx_mesh* m, double* dev, const double* host_in, double* host_out, int nh)
+// One padded field, from its entry (0, 0, 0) of variable 0 on, to a host array
+// [nv][ex][ey][ez] (host_out) or from one (host_in, into dev and, if non-null,
+// dev2); synchronises the stream.  Rows go through the staging buffer in chunks
+// of one copy each.  Where no buffer can be allocated: one 2D copy per variable
+// and x-plane.
+int copy_field(Staging& st, hipStream_t s, const RowField& f, int nv, double* dev, double* dev2,
+               const double* host_in, double* host_out)
 {
-    const Geom& g = m->g;
-    const size_t row = (size_t)g.nz * sizeof(double);
-    for (int v = 0; v < nh; ++v) {
-        for (int x = 0; x < g.nx; ++x) {
-            double* d = dev + (int64_t)v * g.vstride + cell_off(g, x, 0, 0);
-            size_t hoff = ((size_t)v * g.nx + x) * (size_t)g.ny * g.nz;
+    if (host_in == nullptr && host_out == nullptr) return fail(FX_EINVAL, "null host array");
+    std::lock_guard<std::mutex> hold(st.lock);
+    const size_t row = (size_t)f.ez * sizeof(double);
+    const size_t rows = (size_t)nv * f.ex * f.ey;
+    const size_t want = std::min(rows, std::max<size_t>(1, STAGING_BYTES / row)) * row;
+    if (st.cap < want) {
+        FX_HIP(hipStreamSynchronize(s));
+        (void)hipFree(st.buf);
+        st.buf = nullptr;
+        st.cap = 0;
+        if (hipMalloc(&st.buf, want) == hipSuccess) {
+            st.cap = want;
+        } else {
+            st.buf = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+    if (st.buf == nullptr) {
+        for (int v = 0; v < nv; ++v) {
+            for (int x = 0; x < f.ex; ++x) {
+                const int64_t o = v * f.vstride + x * f.sx;
+                const size_t hoff = ((size_t)v * f.ex + x) * (size_t)f.ey * f.ez;
+                const size_t pitch = f.sy * sizeof(double);
+                if (host_in) {
+                    FX_HIP(hipMemcpy2DAsync(dev + o, pitch, host_in + hoff, row, row, f.ey,
+                                            hipMemcpyHostToDevice, s));
+                    if (dev2)
+                        FX_HIP(hipMemcpy2DAsync(dev2 + o, pitch, host_in + hoff, row, row, f.ey,
+                                                hipMemcpyHostToDevice, s));
+                } else {
+                    FX_HIP(hipMemcpy2DAsync(host_out + hoff, row, dev + o, pitch, row, f.ey,
+                                            hipMemcpyDeviceToHost, s));
+                }
+            }
+        }
+    } else {
+        const size_t chunk = st.cap / row;
+        for (size_t r = 0; r < rows; r += chunk) {
+            const size_t n = std::min(chunk, rows - r);
             if (host_in) {
-                FX_HIP(hipMemcpy2DAsync(d, g.sy * sizeof(double), host_in + hoff, row, row, g.ny,
-                                        hipMemcpyHostToDevice, m->stream));
+                FX_HIP(hipMemcpyAsync(st.buf, host_in + r * f.ez, n * row, hipMemcpyHostToDevice, s));
+                FX_HIP(launch_scatter_rows(f, st.buf, dev, dev2, (unsigned)r, (unsigned)n, s));
             } else {
-                FX_HIP(hipMemcpy2DAsync(host_out + hoff, row, d, g.sy * sizeof(double), row, g.ny,
-                                        hipMemcpyDeviceToHost, m->stream));
+                FX_HIP(launch_gather_rows(f, dev, st.buf, (unsigned)r, (unsigned)n, s));
+                FX_HIP(hipMemcpyAsync(host_out + r * f.ez, st.buf, n * row, hipMemcpyDeviceToHost, s));
             }
         }
     }
-    FX_HIP(hipStreamSynchronize(m->stream));
+    FX_HIP(hipStreamSynchronize(s));
     return FX_OK;
 }
 
-int copy_faces(fx_mesh* m, double* dev, double* const* host_in, double* const* host_out)
+// host global [nh][X][Y][Z] <-> device padded cells
+int copy_cells(Staging& st, hipStream_t s, const Geom& g, int nh, double* dev, double* dev2,
+               const double* host_in, double* host_out)
+{
+    const RowField f{g.vstride, g.sx, g.sy, g.nx, g.ny, g.nz};
+    return copy_field(st, s, f, nh, dev + g.origin, dev2 ? dev2 + g.origin : nullptr, host_in,
+                      host_out);
+}
+
+int copy_faces(fx_mesh* m, double* dev, double* dev2, const double* const* host_in,
+               double* const* host_out)
 {
     const Geom& g = m->g;
     for (int d = 0; d < 3; ++d) {
-        int fx_ = g.nx + (d == 0), fy = g.ny + (d == 1), fz = g.nz + (d == 2);
-        const size_t row = (size_t)fz * sizeof(double);
-        for (int x = 0; x < fx_; ++x) {
-            double* dp = dev + (int64_t)d * g.fvstride + cell_off(g, x, 0, 0);
-            size_t hoff = (size_t)x * fy * fz;
-            if (host_in) {
-                FX_HIP(hipMemcpy2DAsync(dp, g.sy * sizeof(double), host_in[d] + hoff, row, row, fy,
-                                        hipMemcpyHostToDevice, m->stream));
-            } else {
-                FX_HIP(hipMemcpy2DAsync(host_out[d] + hoff, row, dp, g.sy * sizeof(double), row, fy,
-                                        hipMemcpyDeviceToHost, m->stream));
-            }
-        }
+        const RowField f{g.fvstride, g.sx, g.sy, g.nx + (d == 0), g.ny + (d == 1), g.nz + (d == 2)};
+        const int64_t o = (int64_t)d * g.fvstride + g.origin;
+        if (int rc = copy_field(m->staging, m->stream, f, 1, dev + o, dev2 ? dev2 + o : nullptr,
+                                host_in ? host_in[d] : nullptr, host_out ? host_out[d] : nullptr))
+            return rc;
     }
-    FX_HIP(hipStreamSynchronize(m->stream));
     return FX_OK;
 }
 
@@ -388,6 +439,7 @@ int fx_mesh_destroy(fx_mesh* m)
         (void)hipFree(m->saved_bf[s]);
     }
     (void)hipFree(m->err);
+    (void)hipFree(m->staging.buf);
     if (m->fork) (void)hipEventDestroy(m->fork);
     if (m->join) (void)hipEventDestroy(m->join);
     if (m->side) (void)hipStreamDestroy(m->side);
@@ -407,8 +459,8 @@ int fx_mesh_set_prim(fx_mesh* m, const double* W)
     if (int rc = check_mesh(m)) return rc;
     if (W == nullptr) return fail(FX_EINVAL, "null W");
     m->cfl_ready = false;
-    for (int s = 0; s < 2; ++s)
-        if (int rc = copy_cells(m, m->W[s], W, nullptr, m->nh)) return rc;
+    if (int rc = copy_cells(m->staging, m->stream, m->g, m->nh, m->W[0], m->W[1], W, nullptr))
+        return rc;
     double zero[2] = {0.0, 0.0};
     FX_HIP(hipMemcpy(m->dev, zero, sizeof(zero), hipMemcpyHostToDevice));
     return FX_OK;
@@ -418,7 +470,7 @@ int fx_mesh_get_prim(fx_mesh* m, int slot, double* W)
 {
     if (int rc = check_mesh(m)) return rc;
     if (W == nullptr || (slot != 0 && slot != 1)) return fail(FX_EINVAL, "bad slot or null W");
-    return copy_cells(m, m->W[slot], nullptr, W, m->nh);
+    return copy_cells(m->staging, m->stream, m->g, m->nh, m->W[slot], nullptr, nullptr, W);
 }
 
 int fx_mesh_set_bf(fx_mesh* m, const double* bx, const double* by, const double* bz)
@@ -426,9 +478,8 @@ int fx_mesh_set_bf(fx_mesh* m, const double* bx, const double* by, const double*
     if (int rc = check_mesh(m)) return rc;
     if (!m->g.mhd) return fail(FX_EINVAL, "mesh has no face fields");
     m->cfl_ready = false;
-    double* in[3] = {(double*)bx, (double*)by, (double*)bz};
-    for (int s = 0; s < 2; ++s)
-        if (int rc = copy_faces(m, m->bf[s], in, nullptr)) return rc;
+    const double* in[3] = {bx, by, bz};
+    if (int rc = copy_faces(m, m->bf[0], m->bf[1], in, nullptr)) return rc;
     // cell B of every slot from the faces (prj_mhd_bf2bc_all)
     for (int s = 0; s < 2; ++s) FX_HIP(launch_bf2bc(m->g, m->W[s], m->bf[s], m->stream));
     FX_HIP(hipStreamSynchronize(m->stream));
@@ -441,7 +492,7 @@ int fx_mesh_get_bf(fx_mesh* m, int slot, double* bx, double* by, double* bz)
     if (!m->g.mhd) return fail(FX_EINVAL, "mesh has no face fields");
     if (slot != 0 && slot != 1) return fail(FX_EINVAL, "bad slot");
     double* out[3] = {bx, by, bz};
-    return copy_faces(m, m->bf[slot], nullptr, out);
+    return copy_faces(m, m->bf[slot], nullptr, nullptr, out);
 }
 
 int fx_calc_dt(fx_mesh* m, double cfl, double* dt)
@@ -775,6 +826,7 @@ struct fx_ensemble {
     // the CFL maxima of the current states are recorded (dev[2] of every
     // instance in the batched schedule, `partial` in the per-instance one)
     bool cfl_ready = false;
+    Staging staging;                     // host transfers
     hipStream_t stream = nullptr;        // owned: graph capture needs a non-null stream
     // schedule: mode 0 = one launch set per instance, 1 = batched
     int mode = 1;
@@ -873,6 +925,7 @@ int fx_ensemble_destroy(fx_ensemble* e)
     (void)hipFree(e->d_queues);
     (void)hipFree(e->dev);
     (void)hipFree(e->partial);
+    (void)hipFree(e->staging.buf);
     if (e->stream) (void)hipStreamDestroy(e->stream);
     delete e;
     return FX_OK;
@@ -980,11 +1033,8 @@ int fx_ensemble_set_prim(fx_ensemble* e, int i, const double* W)
 {
     if (int rc = ens_check(e, i)) return rc;
     e->cfl_ready = false;
-    fx_mesh tmp;
-    tmp.g = e->geoms[i];
-    tmp.stream = e->stream;
-    for (int s = 0; s < 2; ++s)
-        if (int rc = copy_cells(&tmp, e->host_inst[i].W[s], W, nullptr, 6)) return rc;
+    const EnsInst& I = e->host_inst[i];
+    if (int rc = copy_cells(e->staging, e->stream, I.g, 6, I.W[0], I.W[1], W, nullptr)) return rc;
     double zero[4] = {0.0, 0.0, 0.0, 0.0};
     FX_HIP(hipMemcpyAsync(e->host_inst[i].dev, zero, sizeof(zero), hipMemcpyHostToDevice, e->stream));
     FX_HIP(hipStreamSynchronize(e->stream));
@@ -995,10 +1045,8 @@ int fx_ensemble_get_prim(fx_ensemble* e, int i, int slot, double* W)
 {
     if (int rc = ens_check(e, i)) return rc;
     if (slot != 0 && slot != 1) return fail(FX_EINVAL, "bad slot");
-    fx_mesh tmp;
-    tmp.g = e->geoms[i];
-    tmp.stream = e->stream;
-    return copy_cells(&tmp, e->host_inst[i].W[slot], nullptr, W, 6);
+    const EnsInst& I = e->host_inst[i];
+    return copy_cells(e->staging, e->stream, I.g, 6, I.W[slot], nullptr, nullptr, W);
 }
 
 int fx_ensemble_set_schedule(fx_ensemble* e, int mode, int persistent_wgs, int xcd, int table)

@@ -113,6 +113,19 @@ int mhd_ct_split(int64_t nblocks, int ncu);
 // cell-centred B of the active cells from the faces (prj_mhd_bf2bc)
 hipError_t launch_bf2bc(const Geom& g, double* W, const double* bf, hipStream_t s);
 
+// Host transfers of a padded field: the rows [r0, r0 + nrows) of the compact
+// array [nv][ex][ey][ez] that the field's entries from `dev` on stand for
+// (strides vstride, sx, sy, 1), gathered into `buf` or scattered from it; a
+// scatter also writes `dev2` where that is non-null.
+struct RowField {
+    int64_t vstride, sx, sy;
+    int ex, ey, ez;
+};
+hipError_t launch_gather_rows(const RowField& f, const double* dev, double* buf, unsigned r0,
+                              unsigned nrows, hipStream_t s);
+hipError_t launch_scatter_rows(const RowField& f, const double* buf, double* dev, double* dev2,
+                               unsigned r0, unsigned nrows, hipStream_t s);
+
 // CFL time step: dt_out[0] = min(1e99, min over active cells of cfl / denom)
 // times `scale` (the integrator's SSP coefficient); if dt_prev is non-null
 // and *dt_prev > 0, also applies min(dt, factor * dt_prev) and stores the

@@ -3,6 +3,8 @@ oracle.  The mesh sizes are those at which the rules of a 256-CU GPU take each
 number of parts (the edges of the parts fall inside blocks, so a wrong plane at
 a part's edge shows in the cells); bit-identical states and dts, as for whole
 blocks."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -74,3 +76,55 @@ def test_mhd_parts(gpu, n, eta):
         for a, b in zip(gm.get_bf(0), om.bf0):
             assert np.array_equal(a, b)
     gm.close()
+
+
+def _blocks_call(lib, mhd, uniq, n):
+    """fx_flux_update_blocks over n device blocks, copies of the given ones in
+    turn; the outputs as tensors [direction][block]."""
+    import torch
+    from fornaxamr_amd import _native
+    nh = 9 if mhd else 6
+    shapes = {"flux": nh * O.RB_CELLS, "v_riemann": 3 * O.RB_CELLS}
+    if mhd:
+        shapes.update(Bv1=O.RB_CELLS, Bv2=O.RB_CELLS)
+    out = {k: torch.full((3, n, m), float("nan"), dtype=torch.float64, device="cuda")
+           for k, m in shapes.items()}
+    ins = [[torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in (slab, eos, *(bf or []))]
+           for slab, eos, bf in uniq]
+    io = (_native.BlockIO * n)()
+    for b in range(n):
+        own = ins[b % len(ins)]
+        io[b].W, io[b].eosvar, io[b].var_stride = own[0].data_ptr(), own[1].data_ptr(), 2 * O.RB_CELLS
+        for d in range(3):
+            for k in shapes:
+                getattr(io[b], k)[d] = out[k][d, b].data_ptr()
+            if mhd:
+                io[b].bf[d] = own[2 + d].data_ptr()
+    raw = torch.frombuffer(bytearray(bytes(io)), dtype=torch.uint8).cuda()
+    status = torch.zeros(8, dtype=torch.int32, device="cuda")
+    _native.check(lib.fx_flux_update_blocks(n, C.c_void_p(raw.data_ptr()), mhd,
+                                            C.c_void_p(status.data_ptr()),
+                                            C.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    torch.cuda.synchronize()
+    assert status.tolist() == [0] * 8
+    return out
+
+
+@pytest.mark.parametrize("mhd", [0, 1], ids=["hydro", "mhd"])
+def test_block_parts(gpu, mhd):
+    """Per-block fluxes of 1 to 600 blocks in a launch (16 parts down to whole
+    blocks) are those of the first call, whose single blocks the reference's
+    digests pin."""
+    import torch
+    uniq = []
+    for seed in (11, 12, 13):
+        slab, gam, bf = O.block_inputs(seed, bool(mhd))
+        uniq.append((slab, O.block_eosvar(slab, 0, gam), bf))
+    want = _blocks_call(gpu, mhd, uniq, 3)
+    for n in (1, 65, 125, 216, 343, 512, 600):
+        got = _blocks_call(gpu, mhd, uniq, n)
+        for k in want:
+            for b in range(3):
+                ref = want[k][:, b].view(torch.int64)
+                assert all(torch.equal(got[k][:, c].view(torch.int64), ref)
+                           for c in range(b, n, 3)), (n, k, b)

@@ -1194,8 +1194,7 @@ struct fx_adj {
     size_t state_bytes = 0;               // 6 * N doubles
     double* S = nullptr;                  // running state; W_T after a forward
     double* W1 = nullptr;                 // stage-1 output of the plain forward
-    double* F = nullptr;                  // 18 N
-    double* G = nullptr;                  // 36 N
+    double* G = nullptr;                  // 12 N
     double* Ub[2] = {nullptr, nullptr};   // 6 N each
     double* seg = nullptr;                // 2 * every states of one recomputed segment
     double* ckpt = nullptr;               // checkpoints of the last forward
@@ -1221,7 +1220,6 @@ int fx_adj_destroy(fx_adj* a)
     (void)hipDeviceSynchronize();
     (void)hipFree(a->S);
     (void)hipFree(a->W1);
-    (void)hipFree(a->F);
     (void)hipFree(a->G);
     (void)hipFree(a->Ub[0]);
     (void)hipFree(a->Ub[1]);
@@ -1258,8 +1256,7 @@ int fx_adj_create(const int* n, const double* xlim, double gamma, double va_eps2
     a->state_bytes = sizeof(double) * 6 * (size_t)g.N;
     hipError_t e = hipMalloc(&a->S, a->state_bytes);
     if (e == hipSuccess) e = hipMalloc(&a->W1, a->state_bytes);
-    if (e == hipSuccess) e = hipMalloc(&a->F, 3 * a->state_bytes);
-    if (e == hipSuccess) e = hipMalloc(&a->G, 6 * a->state_bytes);
+    if (e == hipSuccess) e = hipMalloc(&a->G, 2 * a->state_bytes);
     if (e == hipSuccess) e = hipMalloc(&a->Ub[0], a->state_bytes);
     if (e == hipSuccess) e = hipMalloc(&a->Ub[1], a->state_bytes);
     if (e == hipSuccess) e = hipMalloc(&a->seg, 2 * (size_t)checkpoint_every * a->state_bytes);
@@ -1287,13 +1284,15 @@ int fx_adj_forward(fx_adj* a, const double* W0, double* WT, int nsteps, double d
         a->ckpt_cap = nck;
     }
     a->nsteps = -1;
-    FX_HIP(hipMemcpyAsync(a->S, W0, a->state_bytes, hipMemcpyDeviceToDevice, s));
+    // each step writes where its result is kept: a checkpoint, or the running state
+    double* X = nsteps > 0 ? a->ckpt : a->S;
+    FX_HIP(hipMemcpyAsync(X, W0, a->state_bytes, hipMemcpyDeviceToDevice, s));
     for (int k = 0; k < nsteps; ++k) {
-        if (k % a->every == 0)
-            FX_HIP(hipMemcpyAsync(adj_state(a->ckpt, a, k / a->every), a->S, a->state_bytes,
-                                  hipMemcpyDeviceToDevice, s));
-        FX_HIP(launch_adj_stage(a->g, 1, dt, a->S, a->S, a->F, a->W1, s));
-        FX_HIP(launch_adj_stage(a->g, 2, dt, a->W1, a->S, a->F, a->S, s));
+        double* out = k + 1 < nsteps && (k + 1) % a->every == 0
+                          ? adj_state(a->ckpt, a, (k + 1) / a->every) : a->S;
+        FX_HIP(launch_adj_stage(a->g, 1, dt, X, X, a->G, a->W1, s));
+        FX_HIP(launch_adj_stage(a->g, 2, dt, a->W1, X, a->G, out, s));
+        X = out;
     }
     FX_HIP(hipMemcpyAsync(WT, a->S, a->state_bytes, hipMemcpyDeviceToDevice, s));
     a->nsteps = nsteps;
@@ -1313,21 +1312,18 @@ int fx_adj_backward(fx_adj* a, const double* gWT, double* gW0, void* stream)
     FX_HIP(launch_adj_w2u(g, a->S, gWT, Ub2, s));
     for (int sg = (n - 1) / K; n > 0 && sg >= 0; --sg) {
         const int k0 = sg * K, k1 = std::min(n, k0 + K), m = k1 - k0;
-        // recompute the segment's stage inputs: seg[2k] = W^n, seg[2k+1] = W^(1)
-        FX_HIP(hipMemcpyAsync(adj_state(a->seg, a, 0), adj_state(a->ckpt, a, sg), a->state_bytes,
-                              hipMemcpyDeviceToDevice, s));
+        // recompute the segment's stage inputs: W^n of step k is state 2k (the
+        // checkpoint for k = 0), W^(1) state 2k + 1
+        auto st = [&](int i) {
+            return i == 0 ? adj_state(a->ckpt, a, sg) : adj_state(a->seg, a, i);
+        };
         for (int k = 0; k < m; ++k) {
-            FX_HIP(launch_adj_stage(g, 1, a->dt, adj_state(a->seg, a, 2 * k),
-                                    adj_state(a->seg, a, 2 * k), a->F,
-                                    adj_state(a->seg, a, 2 * k + 1), s));
+            FX_HIP(launch_adj_stage(g, 1, a->dt, st(2 * k), st(2 * k), a->G, st(2 * k + 1), s));
             if (k + 1 < m)
-                FX_HIP(launch_adj_stage(g, 2, a->dt, adj_state(a->seg, a, 2 * k + 1),
-                                        adj_state(a->seg, a, 2 * k), a->F,
-                                        adj_state(a->seg, a, 2 * k + 2), s));
+                FX_HIP(launch_adj_stage(g, 2, a->dt, st(2 * k + 1), st(2 * k), a->G, st(2 * k + 2), s));
         }
         for (int k = m - 1; k >= 0; --k)
-            FX_HIP(launch_adj_step_reverse(g, a->dt, adj_state(a->seg, a, 2 * k),
-                                           adj_state(a->seg, a, 2 * k + 1), Ub2, Ub1, a->G, s));
+            FX_HIP(launch_adj_step_reverse(g, a->dt, st(2 * k), st(2 * k + 1), Ub2, Ub1, a->G, s));
     }
     // initial state: W0 is checkpoint 0 (or S itself when nsteps == 0)
     const double* W0 = n > 0 ? adj_state(a->ckpt, a, 0) : a->S;

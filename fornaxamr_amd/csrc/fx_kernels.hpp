@@ -194,7 +194,7 @@ struct AdjGeom {
     double eps2;            // van Albada regularisation
 };
 
-// one forward RK2 stage: F scratch 18*N; stage 2 may write Wout == W0
+// one forward RK2 stage: F scratch 12*N; stage 2 may write Wout == W0
 hipError_t launch_adj_stage(const AdjGeom& g, int stage, double dt, const double* Win,
                             const double* W0, double* F, double* Wout, hipStream_t s);
 hipError_t launch_adj_w2u(const AdjGeom& g, const double* W, const double* Wb, double* Ub,
@@ -202,7 +202,7 @@ hipError_t launch_adj_w2u(const AdjGeom& g, const double* W, const double* Wb, d
 hipError_t launch_adj_u2w(const AdjGeom& g, const double* W, const double* Ub, double* Wb,
                           hipStream_t s);
 // reverse of one RK2 step (W0, W1 its stage inputs); U2b in: cotangent of the
-// step's output in conserved form, out: that of W0; U1b 6*N and G 36*N scratch
+// step's output in conserved form, out: that of W0; U1b 6*N and G 12*N scratch
 hipError_t launch_adj_step_reverse(const AdjGeom& g, double dt, const double* W0, const double* W1,
                                    double* U2b, double* U1b, double* G, hipStream_t s);
 

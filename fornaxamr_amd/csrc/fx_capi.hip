@@ -41,7 +41,8 @@ struct fx_mesh {
     double* fdat = nullptr;
     double* zring = nullptr;   // MHD: compact copies of the ghost planes z = -1, nz
     double* dev = nullptr;   // [0] dt, [1] dt_prev, [2] (unused), [3] fx_calc_dt,
-                             // [4] eSSPRK substep dt; from [8] the CFL partials
+                             // [4] eSSPRK substep dt, [5..7] the error word; from
+                             // [8] the CFL partials
     int nblocks = 0;
     // dev + 8 holds cfl_nparts CFL maxima of the current state W[0] (per
     // block for hydro, per CT workgroup for MHD), as recorded by the stage 2
@@ -49,7 +50,7 @@ struct fx_mesh {
     // cfl_ready
     int cfl_nparts = 0;
     bool cfl_ready = false;
-    int* err = nullptr;      // [code, dir, x, y, z, stage]
+    int* err = nullptr;      // [code, dir, x, y, z, stage], in dev[5..7]
     int integrator = FX_RK2;
     int riemann = FX_RIEMANN_HLLC;   // hydro meshes
     int split = 1;           // workgroups per block of the hydro stage / the MHD flux kernel
@@ -127,20 +128,27 @@ int check_mesh(fx_mesh* m)
     return FX_OK;
 }
 
-int read_error_word(fx_mesh* m)
+// Waits for the mesh's stream; *dt, where wanted, is the last device step's, and a
+// recorded error is reported and cleared.  Both come in the one copy that the wait
+// is for (the hydro kernels record no errors: without dt, no copy).
+int sync_mesh(fx_mesh* m, double* dt)
 {
-    int h[6] = {0, 0, 0, 0, 0, 0};
-    FX_HIP(hipMemcpyAsync(h, m->err, sizeof(h), hipMemcpyDeviceToHost, m->stream));
+    double h[8] = {0.0};
+    if (dt != nullptr || m->g.mhd)
+        FX_HIP(hipMemcpyAsync(h, m->dev, sizeof(h), hipMemcpyDeviceToHost, m->stream));
     FX_HIP(hipStreamSynchronize(m->stream));
-    if (h[0] != 0) {
+    int e[6];
+    memcpy(e, h + 5, sizeof(e));
+    if (e[0] != 0) {
         char buf[256];
-        snprintf(buf, sizeof(buf), "%s (stage %d, dir %d, at %d %d %d)", phys_message(h[0]), h[5],
-                 h[1], h[2], h[3], h[4]);
+        snprintf(buf, sizeof(buf), "%s (stage %d, dir %d, at %d %d %d)", phys_message(e[0]), e[5],
+                 e[1], e[2], e[3], e[4]);
         // clear for the next run
         int z[6] = {0, 0, 0, 0, 0, 0};
         FX_HIP(hipMemcpy(m->err, z, sizeof(z), hipMemcpyHostToDevice));
         return fail(FX_EPHYS, buf);
     }
+    if (dt != nullptr) *dt = h[0];
     return FX_OK;
 }
 
@@ -402,8 +410,7 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
         CALC_DT_WGS, (size_t)m->nblocks * (desc->mhd ? std::max(4, m->ct_split) : m->split));
     if (e == hipSuccess) e = hipMalloc(&m->dev, (8 + npart) * sizeof(double));
     if (e == hipSuccess) e = hipMemset(m->dev, 0, 8 * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc(&m->err, 8 * sizeof(int));
-    if (e == hipSuccess) e = hipMemset(m->err, 0, 8 * sizeof(int));
+    m->err = reinterpret_cast<int*>(m->dev + 5);
     if (e != hipSuccess) {
         fx_mesh_destroy(m);
         return fail(e == hipErrorOutOfMemory ? FX_ENOMEM : FX_EHIP,
@@ -438,7 +445,6 @@ int fx_mesh_destroy(fx_mesh* m)
         (void)hipFree(m->saved[s]);
         (void)hipFree(m->saved_bf[s]);
     }
-    (void)hipFree(m->err);
     (void)hipFree(m->staging.buf);
     if (m->fork) (void)hipEventDestroy(m->fork);
     if (m->join) (void)hipEventDestroy(m->join);
@@ -673,16 +679,13 @@ int fx_step_dt(fx_mesh* m, double dt)
 int fx_step(fx_mesh* m, double cfl, double dt_factor, double* dt_used)
 {
     if (int rc = fx_step_async(m, cfl, dt_factor)) return rc;
-    if (int rc = fx_sync(m)) return rc;
-    if (dt_used) return fx_last_dt(m, dt_used);
-    return FX_OK;
+    return sync_mesh(m, dt_used);
 }
 
 int fx_sync(fx_mesh* m)
 {
     if (int rc = check_mesh(m)) return rc;
-    FX_HIP(hipStreamSynchronize(m->stream));
-    return read_error_word(m);
+    return sync_mesh(m, nullptr);
 }
 
 int fx_last_dt(fx_mesh* m, double* dt)

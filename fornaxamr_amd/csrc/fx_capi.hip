@@ -55,15 +55,6 @@ struct fx_mesh {
     int riemann = FX_RIEMANN_HLLC;   // hydro meshes
     int split = 1;           // workgroups per block of the hydro stage / the MHD flux kernel
     int ct_split = 1;        // MHD CT workgroups per block
-    // MHD meshes whose flux kernel fits the chip in one round (at most 2
-    // workgroups per CU): stream and events on which the ghost-layer face
-    // kernel runs beside the flux kernel (default priority, non-blocking).
-    // On larger meshes the flux kernel has every CU busy and the two kernels
-    // run in order (running them together measured 0.4 % slower at 256^3,
-    // 2.7 % faster at 128^3).
-    hipStream_t side = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
-    bool side_on = false;    // the ghost-layer face kernel runs on `side`
     double* saved[2] = {nullptr, nullptr};   // eSSPRK(10,4) saved states u^n, u5
     double* saved_bf[2] = {nullptr, nullptr};   // and their face fields (MHD)
     hipStream_t stream = nullptr;
@@ -245,15 +236,6 @@ int copy_faces(fx_mesh* m, double* dev, double* dev2, const double* const* host_
     return FX_OK;
 }
 
-// the second stream and the fork/join events of the MHD ghost-layer face kernel
-hipError_t create_side_stream(fx_mesh* m)
-{
-    hipError_t e = hipStreamCreateWithFlags(&m->side, hipStreamNonBlocking);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&m->fork, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&m->join, hipEventDisableTiming);
-    return e;
-}
-
 int run_stage(fx_mesh* m, int stage, const double* dt_ptr, double dt)
 {
     const Geom& g = m->g;
@@ -313,8 +295,7 @@ int run_stage(fx_mesh* m, int stage, const double* dt_ptr, double dt)
         FX_HIP(hipEventCreate(&e1));
         FX_HIP(hipEventRecord(e0, m->stream));
     }
-    FX_HIP(launch_mhd_stage(a, stage, m->stream, m->side_on ? m->side : nullptr, m->fork,
-                            m->join));
+    FX_HIP(launch_mhd_stage(a, stage, m->stream));
     m->cfl_ready = stage == 2;
     if (m->timing) {
         FX_HIP(hipEventRecord(e1, m->stream));
@@ -393,14 +374,7 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
     int ncu = 0;
     if (e == hipSuccess) e = cu_count(ncu);
     if (e == hipSuccess) m->split = stage_split(m->nblocks, ncu);
-    if (e == hipSuccess && desc->mhd) {
-        m->ct_split = mhd_ct_split(m->nblocks, ncu);
-        const int64_t nb = m->nblocks;
-        if (nb <= 2 * (int64_t)ncu) {
-            e = create_side_stream(m);
-            m->side_on = e == hipSuccess;
-        }
-    }
+    if (e == hipSuccess && desc->mhd) m->ct_split = mhd_ct_split(m->nblocks, ncu);
     // dev[0..7] scalars, then the CFL partials: one per workgroup of the
     // reduction, or the maxima a stage 2 records
     m->cfl_nparts = m->nblocks * (desc->mhd ? m->ct_split : m->split);
@@ -434,7 +408,6 @@ int fx_mesh_destroy(fx_mesh* m)
     if (m == nullptr) return FX_OK;
     if (m->stream) (void)hipStreamSynchronize(m->stream);
     else (void)hipDeviceSynchronize();
-    if (m->side) (void)hipStreamSynchronize(m->side);
     drop_spans(m);
     for (double* p : m->W) (void)hipFree(p);
     for (double* p : m->bf) (void)hipFree(p);
@@ -446,9 +419,6 @@ int fx_mesh_destroy(fx_mesh* m)
         (void)hipFree(m->saved_bf[s]);
     }
     (void)hipFree(m->staging.buf);
-    if (m->fork) (void)hipEventDestroy(m->fork);
-    if (m->join) (void)hipEventDestroy(m->join);
-    if (m->side) (void)hipStreamDestroy(m->side);
     delete m;
     return FX_OK;
 }
@@ -556,15 +526,11 @@ int fx_mesh_set_mhd_schedule(fx_mesh* m, int ct_split, int side_stream)
     if (side_stream < -1 || side_stream > 1)
         return fail(FX_EINVAL, "side_stream must be -1 (automatic), 0 or 1");
     FX_HIP(hipStreamSynchronize(m->stream));
-    if (m->side) FX_HIP(hipStreamSynchronize(m->side));
     int ncu = 0;
     FX_HIP(cu_count(ncu));
     m->ct_split = ct_split != 0 ? ct_split : mhd_ct_split(m->nblocks, ncu);
     m->cfl_nparts = m->nblocks * m->ct_split;
     m->cfl_ready = false;   // recorded per CT workgroup of the old split
-    bool on = side_stream == 1 || (side_stream == -1 && m->nblocks <= 2 * ncu);
-    if (on && m->side == nullptr) FX_HIP(create_side_stream(m));
-    m->side_on = on;
     return FX_OK;
 }
 

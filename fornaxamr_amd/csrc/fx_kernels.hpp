@@ -101,12 +101,7 @@ hipError_t launch_hydro_stage(const HydroStageArgs& a, int stage, hipStream_t s)
 // blocks on a GPU of ncu CUs
 int stage_split(int64_t nblocks, int ncu);
 
-// side (optional, with the events fork/join): a second stream on which the
-// ghost-layer face kernel runs beside the flux kernel; the CT kernel waits
-// for both.  side == nullptr: all three kernels in order on s.
-hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s,
-                            hipStream_t side = nullptr, hipEvent_t fork = nullptr,
-                            hipEvent_t join = nullptr);
+hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s);
 // CT workgroups per block of a stage over nblocks blocks on a GPU of ncu CUs
 int mhd_ct_split(int64_t nblocks, int ncu);
 

@@ -8,16 +8,17 @@
 // (src/prj_timeint.c:415-495) and the per-cell update with the cell field taken
 // from the new faces (src/prj_timeint.c:498-510, 1255-1350, 1562-1655).
 //
-// Three launches per stage:
+// Two launches per stage after the ghost fill:
 //   mhd_flux_kernel   one workgroup per 16^3 block, marching x-planes like the
 //                     hydro kernel: HLLD on the block's faces, flux divergence,
 //                     RK combination of the hydro conserved variables and their
 //                     conversion to rho, v, Ye and the field-free part of the
 //                     internal energy (into the output slot), and the per-face
-//                     EMF inputs (Bv1, Bv2, normal velocity);
-//   mhd_ghostface_kernel  the same face inputs on the one-face transverse layer
-//                     outside the domain that boundary edges read (the
-//                     reference computes it from ghost cells, -1..16 loops);
+//                     EMF inputs (Bv1, Bv2, normal velocity); further
+//                     workgroups solve the same face inputs on the one-face
+//                     transverse layer outside the domain that boundary edges
+//                     read (the reference computes it from ghost cells, -1..16
+//                     loops);
 //   mhd_ct_kernel     one workgroup per block, marching x-planes: cell EMFs,
 //                     edge EMFs, CT update of the block's faces, cell-centred B
 //                     and the magnetic term of the internal energy.
@@ -125,6 +126,111 @@ __device__ __forceinline__ void store_fdat(const MhdStageArgs& a, int dir, int x
 }
 
 // ---------------------------------------------------------------------------
+// Face EMF inputs on the transverse ghost layer of the domain: faces of
+// direction d whose transverse coordinates include -1 or N (the reference's
+// -1..16 face loops on boundary blocks, src/prj_flux.c:2241-2251).
+__device__ __forceinline__ bool decode_ghostface(const Geom& g, int64_t id64, int& dir, int& x,
+                                                 int& y, int& z)
+{
+    // per direction: normal extent N_d + 1, transverse box (N_t + 2) x (N_u + 2)
+    // minus the inner N_t x N_u.  32-bit unsigned arithmetic: the layer has
+    // about 12 N^2 faces, far below 2^31 for any mesh the C ABI accepts, and
+    // 64-bit division by a run-time divisor is a long software sequence.
+    const int n[3] = {g.nx, g.ny, g.nz};
+    unsigned id = (unsigned)id64;
+    for (int d = 0; d < 3; ++d) {
+        const int t1 = d == 2 ? 0 : d + 1, t2 = d == 0 ? 2 : (d == 1 ? 0 : 1);
+        const unsigned w2 = (unsigned)(n[t2] + 2);
+        const unsigned outer = (unsigned)(n[t1] + 2) * w2;
+        const unsigned ring = outer - (unsigned)n[t1] * (unsigned)n[t2];
+        const unsigned cnt = (unsigned)(n[d] + 1) * ring;
+        if (id < cnt) {
+            // z-faces: the normal index fastest, so that a wave's stencils
+            // (along z) are contiguous; x- and y-faces: the ring position
+            // fastest
+            unsigned nd, r;
+            if (d == 2) {
+                r = id / (unsigned)(n[d] + 1);
+                nd = id - r * (unsigned)(n[d] + 1);
+            } else {
+                nd = id / ring;
+                r = id - nd * ring;
+            }
+            int c1, c2;
+            // ring enumeration: two full rows (c1 = -1, N) then two side columns
+            const unsigned rows = 2u * w2;
+            if (r < rows) {
+                const unsigned hi = r >= w2 ? 1u : 0u;
+                c1 = hi ? n[t1] : -1;
+                c2 = (int)(r - hi * w2) - 1;
+            } else {
+                r -= rows;
+                c1 = (int)(r >> 1);
+                c2 = (r & 1) ? n[t2] : -1;
+            }
+            int c[3];
+            c[d] = (int)nd;
+            c[t1] = c1;
+            c[t2] = c2;
+            dir = d;
+            x = c[0];
+            y = c[1];
+            z = c[2];
+            return true;
+        }
+        id -= cnt;
+    }
+    return false;
+}
+
+__device__ __forceinline__ double bf_clamped(const Geom& g, const double* bf, int dir, int x,
+                                             int y, int z)
+{
+    int hx = g.nx - 1 + (dir == 0), hy = g.ny - 1 + (dir == 1), hz = g.nz - 1 + (dir == 2);
+    x = x < 0 ? 0 : (x > hx ? hx : x);
+    y = y < 0 ? 0 : (y > hy ? hy : y);
+    z = z < 0 ? 0 : (z > hz ? hz : z);
+    return bf[dir * g.fvstride + cell_off(g, x, y, z)];
+}
+
+__device__ __forceinline__ void ghost_face(const MhdStageArgs& a, int64_t id, int stage)
+{
+    int dir, x, y, z;
+    if (!decode_ghostface(a.g, id, dir, x, y, z)) return;
+    const Geom& g = a.g;
+    const double gm1 = g.gamma - 1.0;
+    // the stencil: base (the right cell), the stride along the face normal and
+    // between variables -- in the padded arrays, or, for x- and y-faces on the
+    // ghost planes z = -1 and z = nz, in their compact copies (launch_boundary_fill)
+    int S = dir == 0 ? (int)g.sx : (dir == 1 ? (int)g.sy : 1);
+    const double* base = a.Win + cell_off(g, x, y, z);
+    int64_t vs = g.vstride;
+    if (dir != 2 && (z == -1 || z == g.nz) && a.zring != nullptr) {
+        const int64_t pl = zring_plane(g);
+        const int zc = z == -1 ? 0 : 1;
+        vs = 2 * pl;
+        if (dir == 0) {
+            S = g.ny + 4;
+            base = a.zring + zc * pl + (int64_t)(x + 2) * (g.ny + 4) + (y + 2);
+        } else {
+            S = g.nx + 4;
+            base = a.zring + 18 * pl + zc * pl + (int64_t)(y + 2) * (g.nx + 4) + (x + 2);
+        }
+    }
+    double pq[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const double* cell = base + (s - 2) * S;
+        pq[s] = gm1 * cell[0] * cell[4 * vs];
+    }
+    double bn = bf_clamped(g, a.bf_in, dir, x, y, z);
+    double F6[6], fd3[3];
+    int rc = hlld_face(dir, [&](int v) { return base + v * vs; }, 0, S, pq, g.gamma, bn, F6, fd3);
+    if (rc) set_error(a.err, rc, dir, x, y, z, stage);
+    store_fdat(a, dir, x, y, z, fd3);
+}
+
+// ---------------------------------------------------------------------------
 // Flux kernel.  LDS holds two full planes (x = i and i+1, 20x20 cells with the
 // 2-cell halo, 9 primitives + pressure) so that a thread keeps little state in
 // registers across the HLLD solves: the left state of its next x-face and the
@@ -134,9 +240,21 @@ __device__ __forceinline__ void store_fdat(const MhdStageArgs& a, int dir, int x
 // the block boundary.  The high-side y/z fluxes of a cell come from the
 // neighbouring lanes (shuffles), across wave rows and from the extra faces
 // through a small LDS buffer.
+//
+// Workgroups beyond the nwg of the blocks solve the `ghosts` ghost-layer faces, a
+// set of fdat entries of their own: short ones that fill the last round.  As a
+// launch of its own before this one, or beside it on a second stream, that work
+// cost more at every size (us per step, in order / second stream / here: 8 blocks
+// 112 / 115 / 100, 64 blocks 194 / 215 / 185, 512 blocks 1106 / 1091 / 1077, 4096
+// blocks 7847 / 7892 / 7772).
 template <int STAGE>
-__global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a)
+__global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg, int64_t ghosts)
 {
+    if ((int)blockIdx.x >= nwg) {
+        const int64_t id = (int64_t)((int)blockIdx.x - nwg) * NT + threadIdx.x;
+        if (id < ghosts) ghost_face(a, id, STAGE);
+        return;
+    }
     __shared__ double pl[2][NQ][PC];
     // y-face fluxes that cross a wave boundary: rows 4, 8, 12 (first rows of
     // waves 1-3) and 16 (the block's high-side faces); z-face fluxes at k = 16.
@@ -158,7 +276,7 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a)
     // flux_split workgroups, each marching np planes from x0 with its own
     // prologue; the x-face between two parts is formed by both, from the same
     // cells: identical values
-    const int wg = block_of_workgroup(blockIdx.x, gridDim.x);
+    const int wg = block_of_workgroup(blockIdx.x, nwg);
     const int np = BS / a.flux_split;
     const int part = wg % a.flux_split;
     const int b = wg / a.flux_split;
@@ -396,113 +514,6 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a)
             }
         }
     }
-}
-
-// ---------------------------------------------------------------------------
-// Face EMF inputs on the transverse ghost layer of the domain: faces of
-// direction d whose transverse coordinates include -1 or N (the reference's
-// -1..16 face loops on boundary blocks, src/prj_flux.c:2241-2251).
-__device__ __forceinline__ bool decode_ghostface(const Geom& g, int64_t id64, int& dir, int& x,
-                                                 int& y, int& z)
-{
-    // per direction: normal extent N_d + 1, transverse box (N_t + 2) x (N_u + 2)
-    // minus the inner N_t x N_u.  32-bit unsigned arithmetic: the layer has
-    // about 12 N^2 faces, far below 2^31 for any mesh the C ABI accepts, and
-    // 64-bit division by a run-time divisor is a long software sequence.
-    const int n[3] = {g.nx, g.ny, g.nz};
-    unsigned id = (unsigned)id64;
-    for (int d = 0; d < 3; ++d) {
-        const int t1 = d == 2 ? 0 : d + 1, t2 = d == 0 ? 2 : (d == 1 ? 0 : 1);
-        const unsigned w2 = (unsigned)(n[t2] + 2);
-        const unsigned outer = (unsigned)(n[t1] + 2) * w2;
-        const unsigned ring = outer - (unsigned)n[t1] * (unsigned)n[t2];
-        const unsigned cnt = (unsigned)(n[d] + 1) * ring;
-        if (id < cnt) {
-            // z-faces: the normal index fastest, so that a wave's stencils
-            // (along z) are contiguous; x- and y-faces: the ring position
-            // fastest
-            unsigned nd, r;
-            if (d == 2) {
-                r = id / (unsigned)(n[d] + 1);
-                nd = id - r * (unsigned)(n[d] + 1);
-            } else {
-                nd = id / ring;
-                r = id - nd * ring;
-            }
-            int c1, c2;
-            // ring enumeration: two full rows (c1 = -1, N) then two side columns
-            const unsigned rows = 2u * w2;
-            if (r < rows) {
-                const unsigned hi = r >= w2 ? 1u : 0u;
-                c1 = hi ? n[t1] : -1;
-                c2 = (int)(r - hi * w2) - 1;
-            } else {
-                r -= rows;
-                c1 = (int)(r >> 1);
-                c2 = (r & 1) ? n[t2] : -1;
-            }
-            int c[3];
-            c[d] = (int)nd;
-            c[t1] = c1;
-            c[t2] = c2;
-            dir = d;
-            x = c[0];
-            y = c[1];
-            z = c[2];
-            return true;
-        }
-        id -= cnt;
-    }
-    return false;
-}
-
-__device__ __forceinline__ double bf_clamped(const Geom& g, const double* bf, int dir, int x,
-                                             int y, int z)
-{
-    int hx = g.nx - 1 + (dir == 0), hy = g.ny - 1 + (dir == 1), hz = g.nz - 1 + (dir == 2);
-    x = x < 0 ? 0 : (x > hx ? hx : x);
-    y = y < 0 ? 0 : (y > hy ? hy : y);
-    z = z < 0 ? 0 : (z > hz ? hz : z);
-    return bf[dir * g.fvstride + cell_off(g, x, y, z)];
-}
-
-__global__ void __launch_bounds__(256) mhd_ghostface_kernel(MhdStageArgs a, int64_t total, int stage)
-{
-    const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (id >= total) return;
-    int dir, x, y, z;
-    if (!decode_ghostface(a.g, id, dir, x, y, z)) return;
-    const Geom& g = a.g;
-    const double gm1 = g.gamma - 1.0;
-    // the stencil: base (the right cell), the stride along the face normal and
-    // between variables -- in the padded arrays, or, for x- and y-faces on the
-    // ghost planes z = -1 and z = nz, in their compact copies (launch_boundary_fill)
-    int S = dir == 0 ? (int)g.sx : (dir == 1 ? (int)g.sy : 1);
-    const double* base = a.Win + cell_off(g, x, y, z);
-    int64_t vs = g.vstride;
-    if (dir != 2 && (z == -1 || z == g.nz) && a.zring != nullptr) {
-        const int64_t pl = zring_plane(g);
-        const int zc = z == -1 ? 0 : 1;
-        vs = 2 * pl;
-        if (dir == 0) {
-            S = g.ny + 4;
-            base = a.zring + zc * pl + (int64_t)(x + 2) * (g.ny + 4) + (y + 2);
-        } else {
-            S = g.nx + 4;
-            base = a.zring + 18 * pl + zc * pl + (int64_t)(y + 2) * (g.nx + 4) + (x + 2);
-        }
-    }
-    double pq[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const double* cell = base + (s - 2) * S;
-        pq[s] = gm1 * cell[0] * cell[4 * vs];
-    }
-    double bn = bf_clamped(g, a.bf_in, dir, x, y, z);
-    double F6[6], fd3[3];
-    int rc = hlld_face(dir, [&](int v) { return base + v * vs; }, 0, S, pq, g.gamma, bn, F6, fd3);
-    if (rc) set_error(a.err, rc, dir, x, y, z, stage);
-    store_fdat(a, dir, x, y, z, fd3);
 }
 
 // ---------------------------------------------------------------------------
@@ -847,36 +858,17 @@ int mhd_ct_split(int64_t nblocks, int ncu)
     return split;
 }
 
-hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s, hipStream_t side,
-                            hipEvent_t fork, hipEvent_t join)
+hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s)
 {
     const int nblocks = a.g.nbx * a.g.nby * a.g.nbz;
     if (a.ct_split < 1 || a.ct_split > BS || BS % a.ct_split != 0) return hipErrorInvalidValue;
     if (a.flux_split < 1 || a.flux_split > BS || BS % a.flux_split != 0) return hipErrorInvalidValue;
-    if (side != nullptr && (fork == nullptr || join == nullptr)) return hipErrorInvalidValue;
     const int nfl = nblocks * a.flux_split, nct = nblocks * a.ct_split;
     const int64_t ngf = ghostface_count(a.g);
     if (ngf >= ((int64_t)1 << 31)) return hipErrorInvalidValue;   // 32-bit decode
-    // The ghost-layer faces and the flux kernel's faces are disjoint sets of
-    // fdat entries and both only read the state and the faces: the ghost-layer
-    // kernel (latency-bound, a fraction of the chip) can run beside the flux
-    // kernel (issue-bound at two workgroups per CU).
-    hipStream_t gs = s;
-    if (side != nullptr) {
-        if (hipError_t e = hipEventRecord(fork, s)) return e;
-        if (hipError_t e = hipStreamWaitEvent(side, fork, 0)) return e;
-        gs = side;
-    }
-    hipLaunchKernelGGL(mhd_ghostface_kernel, dim3((unsigned)((ngf + 255) / 256)), dim3(256), 0, gs,
-                       a, ngf, stage);
-    if (side != nullptr) {
-        if (hipError_t e = hipEventRecord(join, side)) return e;
-    }
-    if (stage == 1) hipLaunchKernelGGL(mhd_flux_kernel<1>, dim3(nfl), dim3(NT), 0, s, a);
-    else hipLaunchKernelGGL(mhd_flux_kernel<2>, dim3(nfl), dim3(NT), 0, s, a);
-    if (side != nullptr) {
-        if (hipError_t e = hipStreamWaitEvent(s, join, 0)) return e;
-    }
+    const dim3 grid((unsigned)(nfl + (ngf + NT - 1) / NT));
+    if (stage == 1) hipLaunchKernelGGL(mhd_flux_kernel<1>, grid, dim3(NT), 0, s, a, nfl, ngf);
+    else hipLaunchKernelGGL(mhd_flux_kernel<2>, grid, dim3(NT), 0, s, a, nfl, ngf);
     if (stage == 1) hipLaunchKernelGGL(mhd_ct_kernel<1>, dim3(nct), dim3(NT), 0, s, a);
     else hipLaunchKernelGGL(mhd_ct_kernel<2>, dim3(nct), dim3(NT), 0, s, a);
     return hipGetLastError();

@@ -46,10 +46,7 @@ typedef struct fx_mesh_desc {
  *      single-level mesh: src/prj_mesh.c:1438, src/prj_mesh.c:420) ---------- */
 int fx_mesh_create(const fx_mesh_desc *desc, fx_mesh **out);
 int fx_mesh_destroy(fx_mesh *m);
-/* Stream all launches of this mesh go to (a hipStream_t); NULL = default.
- * An MHD mesh with at most two blocks per CU also runs its ghost-layer face
- * kernel on a stream of its own, forked from and joined back into this one
- * with events within each stage (graph capture follows the fork). */
+/* Stream all launches of this mesh go to (a hipStream_t); NULL = default. */
 int fx_mesh_set_stream(fx_mesh *m, void *hip_stream);
 
 /* ---- state transfer (host arrays in the global layout above) ------------ */
@@ -106,11 +103,10 @@ int fx_mesh_set_integrator(fx_mesh *m, int integrator);
  * option has no reference counterpart.  MHD meshes take HLLD only. */
 /* Launch schedule of an MHD mesh's stage (no reference counterpart; every
  * schedule gives the same bits).  ct_split: CT workgroups per block, 1, 2 or
- * 4 (each marches 16/ct_split of the block's x-planes), 0 automatic (more
- * where the blocks would not fill the chip's CT slots).  side_stream: 1 runs
- * the ghost-layer face kernel on a second stream beside the flux kernel, 0 in
- * order on the mesh's stream, -1 automatic (beside it where the flux kernel
- * fits the chip in one round).  Synchronises the mesh's streams first. */
+ * 4 (each marches 16/ct_split of the block's x-planes), 0 automatic (up to 16
+ * where the blocks would not fill the chip's CT slots).  side_stream: 0, 1 or
+ * -1; the ghost-layer faces run in the flux kernel's launch whichever is given
+ * (1 once meant a second stream).  Synchronises the mesh's stream first. */
 int fx_mesh_set_mhd_schedule(fx_mesh *m, int ct_split, int side_stream);
 #define FX_RIEMANN_HLLC 0
 #define FX_RIEMANN_HLLE 1

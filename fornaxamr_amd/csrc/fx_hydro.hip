@@ -43,22 +43,23 @@ struct PlaneRegs {
     int fo, fh;            // sign flips still to apply (see load_plane)
 };
 
-// Loads one x-plane of the block: the thread's own cell and (has_halo) one
-// halo cell, at offsets already mapped onto active cells.  fo / fh: bit a
+// Loads one x-plane of the block (W: the plane's base, plane_off): the thread's
+// own cell and (has_halo) one halo cell, at byte offsets already mapped onto
+// active cells.  fo / fh: bit a
 // set where the cell stands for a ghost across a reflecting face normal to
 // axis a, whose normal velocity is negated (the values the ghost fill of the
 // reference would hold, src/prj_boundary.c:413-531).  The flips are applied
 // where the values are consumed (flip_plane / store_plane), so that a
 // prefetch does not wait for its loads.
 __device__ __forceinline__ void load_plane(const double* __restrict__ W, int64_t vs,
-                                           int64_t off_own, int64_t off_halo, bool has_halo,
+                                           unsigned own8, unsigned halo8, bool has_halo,
                                            PlaneRegs& r, int fo, int fh)
 {
 #pragma unroll
-    for (int q = 0; q < 6; ++q) r.own[q] = W[q * vs + off_own];
+    for (int q = 0; q < 6; ++q) r.own[q] = at_byte(W + q * vs, own8);
     if (has_halo) {
 #pragma unroll
-        for (int q = 0; q < 6; ++q) r.halo[q] = W[q * vs + off_halo];
+        for (int q = 0; q < 6; ++q) r.halo[q] = at_byte(W + q * vs, halo8);
     }
     r.fo = fo;
     r.fh = fh;
@@ -217,20 +218,19 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
         hym = map_axis(g, 1, g.ny, y0 + hj - NG, hflip);
         hzm = map_axis(g, 2, g.nz, z0 + hk - NG, hflip);
     }
-    const int64_t col_own = cell_off(g, 0, y0 + j, z0 + k);
-    const int64_t col_halo = cell_off(g, 0, hym, hzm);
+    const unsigned own8 = plane_byte(g, y0 + j, z0 + k), halo8 = plane_byte(g, hym, hzm);
 
     // active planes (p in [0, np)): the update and W^n
-    auto own_at = [&](int p) { return col_own + (int64_t)(x0 + p) * g.sx; };
+    auto plane = [&](int p) { return plane_off(g, x0 + p); };
     // plane p of the stencil, mapped; fx receives its x flip bit
     auto plane_x = [&](int p, int& fx) {
         fx = 0;
-        return (int64_t)map_axis(g, 0, g.nx, x0 + p, fx) * g.sx;
+        return plane_off(g, map_axis(g, 0, g.nx, x0 + p, fx));
     };
     auto load_at = [&](int p, PlaneRegs& r) {
         int fx;
         const int64_t xo = plane_x(p, fx);
-        load_plane(Win, vs, col_own + xo, col_halo + xo, has_halo, r, fx, fx | hflip);
+        load_plane(Win + xo, vs, own8, halo8, has_halo, r, fx, fx | hflip);
     };
 
     double Ls[NQ];             // left state of x-face i+1 (rho..ye, p)
@@ -250,12 +250,13 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
         load_at(0, r);
         store_plane(pl[0], r, oidx, hidx, has_halo);        // plane 0
         int fmm, f1;
-        const int64_t omm = col_own + plane_x(-2, fmm), o1 = col_own + plane_x(1, f1);
+        const double* Wmm = Win + plane_x(-2, fmm);
+        const double* W1 = Win + plane_x(1, f1);
 #pragma unroll
         for (int q = 0; q < NV; ++q) {
             c0[q] = r.own[q];
-            cmm[q] = Win[q * vs + omm];
-            c1[q] = Win[q * vs + o1];
+            cmm[q] = at_byte(Wmm + q * vs, own8);
+            c1[q] = at_byte(W1 + q * vs, own8);
         }
         cmm[1] = negate_if(cmm[1], fmm);
         c1[1] = negate_if(c1[1], f1);
@@ -301,10 +302,12 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
     // stage 2: W^n of the own cell of the next plane, loaded an iteration
     // ahead of the update that blends with it
     double w0n[6];
-    if (STAGE == 2) {
+    auto load_w0 = [&](int p) {
+        const double* b = W0 + plane(p);
 #pragma unroll
-        for (int q = 0; q < 6; ++q) w0n[q] = W0[q * vs + own_at(0)];
-    }
+        for (int q = 0; q < 6; ++q) w0n[q] = at_byte(b + q * vs, own8);
+    };
+    if (STAGE == 2) load_w0(0);
 
     for (int i = 0; i < np; ++i) {
         const int A = i & 1;
@@ -522,7 +525,6 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
 
         // ---- per-cell RK2 update -------------------------------------------
         {
-            const int64_t o = own_at(i);
             double u[6], u1[6], w[6];
             if (STAGE == 1) {
                 prim2cons6(wi, u);
@@ -539,8 +541,9 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
                 }
             }
             cons2prim6(u1, w);
+            double* b = Wout + plane(i);
 #pragma unroll
-            for (int v = 0; v < 6; ++v) __builtin_nontemporal_store(w[v], &Wout[v * vs + o]);
+            for (int v = 0; v < 6; ++v) __builtin_nontemporal_store(w[v], &at_byte(b + v * vs, own8));
             if (STAGE == 2) {
                 const double d = cfl_denom(g, w[0], w[1], w[2], w[3], w[4]);
                 if (d > cfl_best) cfl_best = d;   // NaN never wins
@@ -550,10 +553,7 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
 #pragma unroll
         for (int q = 0; q < 6; ++q) Fx[q] = Fxn[q];
         if (i + 3 <= np + 1) load_at(i + 3, pf);
-        if (STAGE == 2 && i + 1 < np) {
-#pragma unroll
-            for (int q = 0; q < 6; ++q) w0n[q] = W0[q * vs + own_at(i + 1)];
-        }
+        if (STAGE == 2 && i + 1 < np) load_w0(i + 1);
     }
     return cfl_best;
 }

@@ -47,6 +47,31 @@ __host__ __device__ inline int64_t cell_off(const Geom& g, int x, int y, int z)
     return g.origin + (int64_t)x * g.sx + (int64_t)y * g.sy + z;
 }
 
+// Plane x of a padded field: a base that a workgroup shares, from which a thread's
+// cells of the plane lie at 32-bit byte offsets (a padded plane has less than 2^32
+// bytes on any mesh the C ABI accepts), so that an access takes its address from
+// scalar registers and one lane offset, without 64-bit lane arithmetic.
+__host__ __device__ inline int64_t plane_off(const Geom& g, int x)
+{
+    return cell_off(g, x, -NG, -PADZ);
+}
+__host__ __device__ inline unsigned plane_byte(const Geom& g, int y, int z)
+{
+    return ((unsigned)(y + NG) * (unsigned)g.sy + (unsigned)(z + PADZ)) * 8u;
+}
+// The empty asm keeps the offset from being folded into a loop-invariant 64-bit
+// lane address, which the compiler would otherwise form and add to.
+__device__ __forceinline__ const double& at_byte(const double* base, unsigned byte)
+{
+    asm("" : "+v"(byte));
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + byte);
+}
+__device__ __forceinline__ double& at_byte(double* base, unsigned byte)
+{
+    asm("" : "+v"(byte));
+    return *reinterpret_cast<double*>(reinterpret_cast<char*>(base) + byte);
+}
+
 // Ghost mapping of one axis: the active cell a ghost coordinate c stands for
 // -- periodic wrap (the wrapped neighbour of src/prj_mesh.c:1597-1645) or the
 // mirror copy of the physical boundary (src/prj_boundary.c:413-487: src =

@@ -303,15 +303,15 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
         hk = c < 2 ? c : c + BS;
     }
     const int hidx = hj * PW + hk;
-    const int64_t col_own = cell_off(g, x0, y0 + j, z0 + k);
-    const int64_t col_halo = cell_off(g, x0, y0 + hj - NG, z0 + hk - NG);
-    auto own_at = [&](int p) { return col_own + (int64_t)p * g.sx; };
-    auto halo_at = [&](int p) { return col_halo + (int64_t)p * g.sx; };
+    const unsigned own8 = plane_byte(g, y0 + j, z0 + k),
+                   halo8 = plane_byte(g, y0 + hj - NG, z0 + hk - NG);
+    auto plane = [&](int p) { return plane_off(g, x0 + p); };
 
     // own cell of plane p: 9 primitives and the pressure
     auto load_own = [&](int p, double* c) {
+        const double* b = a.Win + plane(p);
 #pragma unroll
-        for (int q = 0; q < 9; ++q) c[q] = a.Win[q * vs + own_at(p)];
+        for (int q = 0; q < 9; ++q) c[q] = at_byte(b + q * vs, own8);
         c[9] = gm1 * c[0] * c[4];
     };
     // plane p into LDS slot s: the own cell given, the halo cell loaded here
@@ -320,8 +320,9 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
         for (int q = 0; q < NQ; ++q) pl[s][q][oidx] = own[q];
         if (has_halo) {
             double h[9];
+            const double* b = a.Win + plane(p);
 #pragma unroll
-            for (int q = 0; q < 9; ++q) h[q] = a.Win[q * vs + halo_at(p)];
+            for (int q = 0; q < 9; ++q) h[q] = at_byte(b + q * vs, halo8);
 #pragma unroll
             for (int q = 0; q < 9; ++q) pl[s][q][hidx] = h[q];
             pl[s][9][hidx] = gm1 * h[0] * h[4];
@@ -343,7 +344,7 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
             if (q < 9) { WL[q] = Ls[q]; WR[q] = r; } else { pL = Ls[9]; pR = r; }
             Ls[q] = c1[q] + h;
         }
-        double bn = a.bf_in[cell_off(g, x0 + xf, y0 + j, z0 + k)];
+        double bn = at_byte(a.bf_in + plane(xf), own8);
         WL[B1] = bn;
         WR[B1] = bn;
         double Fl[9], vf[3], bv1 = 0.0, bv2 = 0.0;
@@ -351,8 +352,10 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
         if (rc) set_error(a.err, rc, 0, x0 + xf, y0 + j, z0 + k, STAGE);
 #pragma unroll
         for (int v = 0; v < 6; ++v) F6[v] = Fl[v];
-        double fd3[3] = {bv1, bv2, vf[0]};
-        store_fdat(a, 0, x0 + xf, y0 + j, z0 + k, fd3);
+        double* fd = a.fdat + plane(xf);
+        at_byte(fd, own8) = bv1;
+        at_byte(fd + vs, own8) = bv2;
+        at_byte(fd + 2 * vs, own8) = vf[0];
     };
 
     // ---- prologue: planes 0, 1 into LDS; x-face 0 -------------------------
@@ -439,14 +442,16 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
         // divergence and update below (it goes to LDS at the end of the plane)
         double hh[9];
         if (has_halo && i < np - 1) {
+            const double* b = a.Win + plane(i + 2);
 #pragma unroll
-            for (int q = 0; q < 9; ++q) hh[q] = a.Win[q * vs + halo_at(i + 2)];
+            for (int q = 0; q < 9; ++q) hh[q] = at_byte(b + q * vs, halo8);
         }
         // stage 2: W^n of the own cell, for the RK combination below
         double w0[9];
         if (STAGE == 2) {
+            const double* b = a.W0 + plane(i);
 #pragma unroll
-            for (int q = 0; q < 9; ++q) w0[q] = a.W0[q * vs + own_at(i)];
+            for (int q = 0; q < 9; ++q) w0[q] = at_byte(b + q * vs, own8);
         }
 
         // ---- divergence (x, y, z order) and the RK combination -------------
@@ -497,9 +502,9 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
                 w[4] = u1[4] / rho - kinetic;
                 w[5] = u1[5] / rho;
             }
-            const int64_t o = own_at(i);
+            double* b = a.Wout + plane(i);
 #pragma unroll
-            for (int v = 0; v < 6; ++v) a.Wout[v * vs + o] = w[v];
+            for (int v = 0; v < 6; ++v) at_byte(b + v * vs, own8) = w[v];
         }
 #pragma unroll
         for (int v = 0; v < 6; ++v) Fx[v] = Fxn[v];

@@ -482,19 +482,17 @@ __device__ __forceinline__ double emf_upwind(const double* ef, const double* ec,
 // log(DBL_MAX) < 710, so the mask stays below 1e12 * 710^2.  The quotients
 // are formed only past the thresholds: rounding is monotone, so rho <= 1e13
 // gives rho / 1e13 <= 1 (and ye / 0.25 is exact), and the factors are 0
-// there without a division.
+// there without a division.  A factor of 0 makes the mask 0 (the other is finite),
+// so the logs are taken only where both are positive, by one copy of the code.
 __device__ __forceinline__ double eta_mask(double rho, double ye)
 {
-    double rf = 0.0, yf = 0.0;
-    if (rho > 1.0e13 && isfinite(rho)) {
-        double a = rho / 1.0e13;
-        if (a > 1.0) rf = log_cr(a);
-    }
-    if (ye > 0.25 && isfinite(ye)) {
-        double b = ye / 0.25;
-        if (b > 1.0) yf = log_cr(b);
-    }
-    return 1.0e12 * rf * yf;
+    if (!(rho > 1.0e13 && isfinite(rho) && ye > 0.25 && isfinite(ye))) return 0.0;
+    const double x[2] = {rho / 1.0e13, ye / 0.25};
+    double f[2] = {0.0, 0.0};
+#pragma unroll 1
+    for (int n = 0; n < 2; ++n)
+        if ((n == 0 ? x[0] : x[1]) > 1.0) (n == 0 ? f[0] : f[1]) = log_cr(n == 0 ? x[0] : x[1]);
+    return 1.0e12 * f[0] * f[1];
 }
 
 }  // namespace fx

@@ -367,7 +367,7 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
             e = hipMalloc(&m->bf[s], 3 * m->cell_bytes);
             if (e == hipSuccess) e = hipMemset(m->bf[s], 0, 3 * m->cell_bytes);
         }
-        if (e == hipSuccess) e = hipMalloc(&m->fdat, 9 * m->cell_bytes);
+        if (e == hipSuccess) e = hipMalloc(&m->fdat, fdat_doubles(m->g) * sizeof(double));
         if (e == hipSuccess) e = hipMalloc(&m->zring, zring_doubles(m->g) * sizeof(double));
     }
     m->nblocks = m->g.nbx * m->g.nby * m->g.nbz;

@@ -33,7 +33,8 @@ struct MhdStageArgs {
     const double* bf_in;    // face fields of the stage input (3 components)
     const double* bf0;      // face fields at t^n (stage-2 blend)
     double* bf_out;
-    double* fdat;           // scratch: face EMFs and normal velocities (3 dirs x 3)
+    double* fdat;           // scratch (fdat_doubles): face EMFs (3 dirs x 2), then the sign
+                            // words of the normal velocities (3 dirs)
     const double* zring;    // compact copies of the ghost planes z = -1, nz (zring_doubles)
     int* err;               // device error word: [code, dir, x, y, z]
     const double* dt_ptr;
@@ -74,6 +75,12 @@ hipError_t launch_ens_dt_finalize(const EnsInst* inst, int ninst, double cfl, do
 hipError_t launch_ens_stage(const EnsInst* inst, const EnsBlock* blocks, int nblocks, int stage,
                             int split, int persistent_wgs, int xcd_remap, int xcd_queues,
                             int* queues, hipStream_t s);
+
+// MHD scratch of a mesh: 6 fields of doubles and 3 of 32-bit words
+__host__ __device__ inline int64_t fdat_doubles(const Geom& g)
+{
+    return 6 * g.vstride + (3 * g.vstride + 1) / 2;
+}
 
 // Compact copies of the MHD ghost planes z = -1 and z = nz (the 9 cell
 // variables over x, y in [-2, n + 2)), which the ghost-layer face kernel reads

@@ -66,10 +66,11 @@ __device__ __forceinline__ const double& at_byte(const double* base, unsigned by
     asm("" : "+v"(byte));
     return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(base) + byte);
 }
-__device__ __forceinline__ double& at_byte(double* base, unsigned byte)
+template <typename T>
+__device__ __forceinline__ T& at_byte(T* base, unsigned byte)
 {
     asm("" : "+v"(byte));
-    return *reinterpret_cast<double*>(reinterpret_cast<char*>(base) + byte);
+    return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + byte);
 }
 
 // Ghost mapping of one axis: the active cell a ghost coordinate c stands for

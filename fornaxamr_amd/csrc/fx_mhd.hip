@@ -117,12 +117,23 @@ __device__ __forceinline__ int hlld_face(int dir, const Rows& rows, int c, int S
     return rc;
 }
 
+// face EMFs (comp 0, 1) and sign words of the normal velocity, per direction
+__device__ __forceinline__ double* fdat_emf(const MhdStageArgs& a, int dir, int comp)
+{
+    return a.fdat + (dir * 2 + comp) * a.g.vstride;
+}
+__device__ __forceinline__ SignWord* fdat_sign(const MhdStageArgs& a, int dir)
+{
+    return reinterpret_cast<SignWord*>(a.fdat + 6 * a.g.vstride) + dir * a.g.vstride;
+}
+
 __device__ __forceinline__ void store_fdat(const MhdStageArgs& a, int dir, int x, int y, int z,
                                            const double* fd3)
 {
     const int64_t o = cell_off(a.g, x, y, z);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) a.fdat[(dir * 3 + c) * a.g.vstride + o] = fd3[c];
+    fdat_emf(a, dir, 0)[o] = fd3[0];
+    fdat_emf(a, dir, 1)[o] = fd3[1];
+    fdat_sign(a, dir)[o] = sign_word(fd3[2]);
 }
 
 // ---------------------------------------------------------------------------
@@ -352,10 +363,9 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
         if (rc) set_error(a.err, rc, 0, x0 + xf, y0 + j, z0 + k, STAGE);
 #pragma unroll
         for (int v = 0; v < 6; ++v) F6[v] = Fl[v];
-        double* fd = a.fdat + plane(xf);
-        at_byte(fd, own8) = bv1;
-        at_byte(fd + vs, own8) = bv2;
-        at_byte(fd + 2 * vs, own8) = vf[0];
+        at_byte(fdat_emf(a, 0, 0) + plane(xf), own8) = bv1;
+        at_byte(fdat_emf(a, 0, 1) + plane(xf), own8) = bv2;
+        at_byte(fdat_sign(a, 0) + plane(xf), own8 >> 1) = sign_word(vf[0]);
     };
 
     // ---- prologue: planes 0, 1 into LDS; x-face 0 -------------------------
@@ -530,7 +540,11 @@ constexpr int EW = BS + 1;           // 17
 __device__ __forceinline__ double fdat_at(const MhdStageArgs& a, int dir, int comp, int x, int y,
                                           int z)
 {
-    return a.fdat[(dir * 3 + comp) * a.g.vstride + cell_off(a.g, x, y, z)];
+    return fdat_emf(a, dir, comp)[cell_off(a.g, x, y, z)];
+}
+__device__ __forceinline__ SignWord sign_at(const MhdStageArgs& a, int dir, int x, int y, int z)
+{
+    return fdat_sign(a, dir)[cell_off(a.g, x, y, z)];
 }
 
 // resistive curl B at an edge (src/prj_mhd.c:689-711), faces of the stage input
@@ -603,9 +617,9 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
     auto cidx = [](int cj, int ck) { return (cj + 1) * CW + (ck + 1); };
     // one edge EMF from gathered inputs
     auto edge = [&](int dir, int gx, int gy, int gz, const double* ef, const double* ec,
-                    const double* vn, const double* mk) -> double {
+                    const SignWord* vn, const double* mk) -> double {
         for (int n = 0; n < 4; ++n) {
-            if (!isfinite(ef[n]) || !isfinite(ec[n]) || !isfinite(vn[n])) {
+            if (!isfinite(ef[n]) || !isfinite(ec[n]) || !is_finite(vn[n])) {
                 set_error(a.err, 33, dir, gx, gy, gz, STAGE);
             }
         }
@@ -620,15 +634,16 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
     // Ey at x-position X (local), (j, k) with j 0..15, k 0..16; cell planes X-1 (slot sm), X (slot s0)
     auto edge_y = [&](int X, int jj, int kk, int sm, int s0) -> double {
         const int gx = x0 + X, gy = y0 + jj, gz = z0 + kk;
-        double ef[4], ec[4], vn[4], mk[4];
+        double ef[4], ec[4], mk[4];
+        SignWord vn[4];
         ef[0] = fdat_at(a, 0, 0, gx, gy, gz);
         ef[1] = fdat_at(a, 2, 1, gx, gy, gz);
         ef[2] = fdat_at(a, 0, 0, gx, gy, gz - 1);
         ef[3] = fdat_at(a, 2, 1, gx - 1, gy, gz);
-        vn[0] = fdat_at(a, 0, 2, gx, gy, gz);
-        vn[1] = fdat_at(a, 2, 2, gx, gy, gz);
-        vn[2] = fdat_at(a, 0, 2, gx, gy, gz - 1);
-        vn[3] = fdat_at(a, 2, 2, gx - 1, gy, gz);
+        vn[0] = sign_at(a, 0, gx, gy, gz);
+        vn[1] = sign_at(a, 2, gx, gy, gz);
+        vn[2] = sign_at(a, 0, gx, gy, gz - 1);
+        vn[3] = sign_at(a, 2, gx - 1, gy, gz);
         const int c0 = cidx(jj, kk), c1 = cidx(jj, kk - 1);
         ec[0] = ce[s0][1][c0]; mk[0] = ce[s0][3][c0];
         ec[1] = ce[s0][1][c1]; mk[1] = ce[s0][3][c1];
@@ -639,15 +654,16 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
     // Ez at x-position X, (j, k) with j 0..16, k 0..15
     auto edge_z = [&](int X, int jj, int kk, int sm, int s0) -> double {
         const int gx = x0 + X, gy = y0 + jj, gz = z0 + kk;
-        double ef[4], ec[4], vn[4], mk[4];
+        double ef[4], ec[4], mk[4];
+        SignWord vn[4];
         ef[0] = fdat_at(a, 1, 0, gx, gy, gz);
         ef[1] = fdat_at(a, 0, 1, gx, gy, gz);
         ef[2] = fdat_at(a, 1, 0, gx - 1, gy, gz);
         ef[3] = fdat_at(a, 0, 1, gx, gy - 1, gz);
-        vn[0] = fdat_at(a, 1, 2, gx, gy, gz);
-        vn[1] = fdat_at(a, 0, 2, gx, gy, gz);
-        vn[2] = fdat_at(a, 1, 2, gx - 1, gy, gz);
-        vn[3] = fdat_at(a, 0, 2, gx, gy - 1, gz);
+        vn[0] = sign_at(a, 1, gx, gy, gz);
+        vn[1] = sign_at(a, 0, gx, gy, gz);
+        vn[2] = sign_at(a, 1, gx - 1, gy, gz);
+        vn[3] = sign_at(a, 0, gx, gy - 1, gz);
         const int c0 = cidx(jj, kk), c3 = cidx(jj - 1, kk);
         ec[0] = ce[s0][2][c0]; mk[0] = ce[s0][3][c0];
         ec[1] = ce[sm][2][c0]; mk[1] = ce[sm][3][c0];
@@ -658,15 +674,16 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
     // Ex in plane i (local), (j, k) with j, k 0..16; cells in slot s
     auto edge_x = [&](int i, int jj, int kk, int s) -> double {
         const int gx = x0 + i, gy = y0 + jj, gz = z0 + kk;
-        double ef[4], ec[4], vn[4], mk[4];
+        double ef[4], ec[4], mk[4];
+        SignWord vn[4];
         ef[0] = fdat_at(a, 2, 0, gx, gy, gz);
         ef[1] = fdat_at(a, 1, 1, gx, gy, gz);
         ef[2] = fdat_at(a, 2, 0, gx, gy - 1, gz);
         ef[3] = fdat_at(a, 1, 1, gx, gy, gz - 1);
-        vn[0] = fdat_at(a, 2, 2, gx, gy, gz);
-        vn[1] = fdat_at(a, 1, 2, gx, gy, gz);
-        vn[2] = fdat_at(a, 2, 2, gx, gy - 1, gz);
-        vn[3] = fdat_at(a, 1, 2, gx, gy, gz - 1);
+        vn[0] = sign_at(a, 2, gx, gy, gz);
+        vn[1] = sign_at(a, 1, gx, gy, gz);
+        vn[2] = sign_at(a, 2, gx, gy - 1, gz);
+        vn[3] = sign_at(a, 1, gx, gy, gz - 1);
         const int c0 = cidx(jj, kk), c1 = cidx(jj - 1, kk), c2 = cidx(jj - 1, kk - 1),
                   c3 = cidx(jj, kk - 1);
         ec[0] = ce[s][0][c0]; mk[0] = ce[s][3][c0];

@@ -454,21 +454,41 @@ __device__ __forceinline__ int hlld(const double* WL, const double* WR, double p
     return HLLD_OK;
 }
 
+// What the CT step needs of a double in 32 bits: its sign, whether it is zero and
+// whether it is finite.  The high word, with its lowest bit set where the low word
+// is not zero, so that no nonzero value looks like zero.
+struct SignWord {
+    int w;
+};
+__device__ __forceinline__ SignWord sign_word(double v)
+{
+    const long long b = __double_as_longlong(v);
+    return {(int)(b >> 32) | ((int)b != 0 ? 1 : 0)};
+}
+__device__ __forceinline__ bool is_positive(double v) { return v > 0.0; }
+__device__ __forceinline__ bool is_negative(double v) { return v < 0.0; }
+// (of finite values; a word that is not finite is reported before its sign matters)
+__device__ __forceinline__ bool is_positive(SignWord v) { return v.w > 0; }
+__device__ __forceinline__ bool is_negative(SignWord v) { return (unsigned)v.w > 0x80000000u; }
+__device__ __forceinline__ bool is_finite(SignWord v) { return (v.w & 0x7ff00000) != 0x7ff00000; }
+
 // Upwind CT edge EMF without the resistive term (src/prj_mhd.c:651-683).
-__device__ __forceinline__ double emf_upwind(const double* ef, const double* ec, const double* vn)
+// The normal velocities enter by their signs only: V is double, or SignWord.
+template <typename V>
+__device__ __forceinline__ double emf_upwind(const double* ef, const double* ec, const V* vn)
 {
     double emf = 0.25 * (ef[0] + ef[1] + ef[2] + ef[3]);
-    if (vn[0] > 0.0)      emf += 0.25 * (ef[3] - ec[3]);
-    else if (vn[0] < 0.0) emf += 0.25 * (ef[1] - ec[0]);
+    if (is_positive(vn[0]))      emf += 0.25 * (ef[3] - ec[3]);
+    else if (is_negative(vn[0])) emf += 0.25 * (ef[1] - ec[0]);
     else                  emf += 0.125 * (ef[3] - ec[3] + ef[1] - ec[0]);
-    if (vn[1] > 0.0)      emf += 0.25 * (ef[2] - ec[1]);
-    else if (vn[1] < 0.0) emf += 0.25 * (ef[0] - ec[0]);
+    if (is_positive(vn[1]))      emf += 0.25 * (ef[2] - ec[1]);
+    else if (is_negative(vn[1])) emf += 0.25 * (ef[0] - ec[0]);
     else                  emf += 0.125 * (ef[2] - ec[1] + ef[0] - ec[0]);
-    if (vn[2] > 0.0)      emf += 0.25 * (ef[3] - ec[2]);
-    else if (vn[2] < 0.0) emf += 0.25 * (ef[1] - ec[1]);
+    if (is_positive(vn[2]))      emf += 0.25 * (ef[3] - ec[2]);
+    else if (is_negative(vn[2])) emf += 0.25 * (ef[1] - ec[1]);
     else                  emf += 0.125 * (ef[3] - ec[2] + ef[1] - ec[1]);
-    if (vn[3] > 0.0)      emf += 0.25 * (ef[2] - ec[2]);
-    else if (vn[3] < 0.0) emf += 0.25 * (ef[0] - ec[3]);
+    if (is_positive(vn[3]))      emf += 0.25 * (ef[2] - ec[2]);
+    else if (is_negative(vn[3])) emf += 0.25 * (ef[0] - ec[3]);
     else                  emf += 0.125 * (ef[2] - ec[2] + ef[0] - ec[3]);
     return emf;
 }

@@ -146,13 +146,22 @@ hipError_t launch_dt_reduce(const Geom& g, const double* W, double* partial, int
                             hipStream_t s);
 hipError_t launch_dt_final(const double* partial, int n, double cfl, double* dt_out,
                            double* dt_prev, double factor, double scale, hipStream_t s);
-// eSSPRK convex blend of the active cells: W <- prim(w u(Ws) + (1 - w) u(W))
-hipError_t launch_blend(const Geom& g, double* W, const double* Ws, double saved_weight,
-                        hipStream_t s);
-// the same on an MHD mesh: the face fields first (bf <- w bfs + (1 - w) bf),
-// then the cells with their field from the blended faces
-hipError_t launch_blend_mhd(const Geom& g, double* W, const double* Ws, double* bf,
-                            const double* bfs, double saved_weight, hipStream_t s);
+// eSSPRK convex blend of the active cells: dst <- prim(w u(Ws) + (1 - w) u(W))
+hipError_t launch_blend(const Geom& g, const double* W, const double* Ws, double saved_weight,
+                        double* dst, hipStream_t s);
+// two of them, one after the other: W' = the blend of W with Ws, then
+// dst <- the blend of W' with dst (weights w and wd)
+hipError_t launch_blend2(const Geom& g, const double* W, const double* Ws, double saved_weight,
+                         double* dst, double dst_weight, hipStream_t s);
+// the same on an MHD mesh: the face fields first (dst_bf <- w bfs + (1 - w) bf),
+// then the cells with their field from the blended faces; the pair leaves the
+// faces of its first blend in bf
+hipError_t launch_blend_mhd(const Geom& g, const double* W, double* bf, const double* Ws,
+                            const double* bfs, double saved_weight, double* dst, double* dst_bf,
+                            hipStream_t s);
+hipError_t launch_blend2_mhd(const Geom& g, const double* W, double* bf, const double* Ws,
+                             const double* bfs, double saved_weight, double* dst,
+                             double* dst_bf, double dst_weight, hipStream_t s);
 // dst[0] = src[0] / div on the device
 hipError_t launch_div_scalar(const double* src, double* dst, double div, hipStream_t s);
 

@@ -122,8 +122,8 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
     const int x0 = (wg % split) * np;
     const int x1 = x0 + np == BS ? BS + 1 : x0 + np;   // the last part adds x-face 16
     const int64_t vs = bp->var_stride;
-    const double* __restrict__ W = bp->W;
-    const double* __restrict__ eos = bp->eosvar;
+    const double* __restrict__ W = as_global(bp->W);
+    const double* __restrict__ eos = as_global(bp->eosvar);
 
     // own cell and (t < 144) one halo cell of the 20 x 20 plane
     const int oidx = (j + RNG) * RB + (k + RNG);
@@ -144,11 +144,13 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
 
     struct Cell { double q[NQ]; };
     auto load_cell = [&](int p, int c, int e, Cell& r) {
-        const int o = (p + RNG) * PC + c, x = (p + RNG) * (PC * 3) + e;
+        // scalar plane base + 32-bit lane offset
+        const double* Wp = W + (p + RNG) * PC;
+        const double* Ep = eos + (p + RNG) * (PC * 3);
 #pragma unroll
-        for (int q = 0; q < 6; ++q) r.q[q] = W[q * vs + o];
-        r.q[6] = eos[x];
-        r.q[7] = eos[x + 2 * AW];
+        for (int q = 0; q < 6; ++q) r.q[q] = at_byte(Wp + q * vs, 8u * c);
+        r.q[6] = at_byte(Ep, 8u * e);
+        r.q[7] = at_byte(Ep + 2 * AW, 8u * e);
     };
     auto load_plane = [&](int p, Cell& own, Cell& halo) {
         load_cell(p, oidx, eo, own);
@@ -183,8 +185,8 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
     const int krow = ((lane >> 4) * SFP) + k, vrow = ((lane >> 4) * SVP) + k;
     // fluxes and face velocities of this thread's face (i, j, k) of direction dir
     auto put = [&](int dir, int i, const double* Fl, const double* vl) {
-        double* F = bp->flux[dir];
-        double* vr = bp->v_riemann[dir];
+        double* F = as_global(bp->flux[dir]);
+        double* vr = as_global(bp->v_riemann[dir]);
         // paired 16-byte stores where the arrays lie on 16-byte boundaries
         if (((reinterpret_cast<uintptr_t>(F) | reinterpret_cast<uintptr_t>(vr)) & 15) == 0) {
             double* sf = L.f[wave];
@@ -202,10 +204,13 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
             vr += i * (RB * RB * 3);
 #pragma unroll
             for (int s = 0; s < 3; ++s)
-                *reinterpret_cast<double2*>(&F[fdst[s]]) = *reinterpret_cast<const double2*>(&sf[fsrc[s]]);
-            *reinterpret_cast<double2*>(&vr[vdst[0]]) = *reinterpret_cast<const double2*>(&sv[vsrc[0]]);
+                at_byte(reinterpret_cast<double2*>(F), 8u * fdst[s]) =
+                    *reinterpret_cast<const double2*>(&sf[fsrc[s]]);
+            at_byte(reinterpret_cast<double2*>(vr), 8u * vdst[0]) =
+                *reinterpret_cast<const double2*>(&sv[vsrc[0]]);
             if (lane < 32)
-                *reinterpret_cast<double2*>(&vr[vdst[1]]) = *reinterpret_cast<const double2*>(&sv[vsrc[1]]);
+                at_byte(reinterpret_cast<double2*>(vr), 8u * vdst[1]) =
+                    *reinterpret_cast<const double2*>(&sv[vsrc[1]]);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -328,8 +333,8 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
             if (f < 3) {
                 put(f, i, Fl, vl);
             } else {
-                double* F = dir == 1 ? bp->flux[1] : bp->flux[2];
-                double* vr = dir == 1 ? bp->v_riemann[1] : bp->v_riemann[2];
+                double* F = dir == 1 ? as_global(bp->flux[1]) : as_global(bp->flux[2]);
+                double* vr = dir == 1 ? as_global(bp->v_riemann[1]) : as_global(bp->v_riemann[2]);
                 const double g1 = dir == 1 ? Fl[3] : Fl[2], g2 = dir == 1 ? Fl[1] : Fl[3],
                              g3 = dir == 1 ? Fl[2] : Fl[1];
                 double* Fo = F + bidx(6, 0, i, fj, fk);
@@ -400,15 +405,17 @@ __global__ void __launch_bounds__(NTM, 1) block_march_mhd_kernel(const fx_block_
         const int hi = (int)min((int64_t)(MP - 1), lo + (end - at));
         at += hi - lo;
         const int64_t vs = bp->var_stride;
-        const double* __restrict__ W = bp->W;
-        const double* __restrict__ eos = bp->eosvar;
+        const double* __restrict__ W = as_global(bp->W);
+        const double* __restrict__ eos = as_global(bp->eosvar);
 
         auto load_cell = [&](int p, double* q) {
-            const int o = (p + RNG) * PC + t, x = (p + RNG) * (PC * 3) + eo;
+            // scalar plane base + 32-bit lane offset
+            const double* Wp = W + (p + RNG) * PC;
+            const double* Ep = eos + (p + RNG) * (PC * 3);
 #pragma unroll
-            for (int v = 0; v < 9; ++v) q[v] = W[v * vs + o];
-            q[9] = eos[x];
-            q[10] = eos[x + 2 * AW];
+            for (int v = 0; v < 9; ++v) q[v] = at_byte(Wp + v * vs, 8u * t);
+            q[9] = at_byte(Ep, 8u * eo);
+            q[10] = at_byte(Ep + 2 * AW, 8u * eo);
         };
         auto store_cell = [&](int p, const double* q) {
             double* s = lds + (p & 3) * (NQ * PC) + t;
@@ -440,7 +447,7 @@ __global__ void __launch_bounds__(NTM, 1) block_march_mhd_kernel(const fx_block_
                 const int n = dir == 0 ? (BS + 2) * (BS + 2) : (BS + 1) * (BS + 2);
                 if (e >= n || (dir == 0 && i < 0)) continue;
                 const int j = e / w - (dir != 1), k = e - e / w * w - (dir != 2);
-                const double bn = bp->bf[dir][face_idx(dir, i, j, k)];
+                const double bn = as_global(bp->bf[dir])[face_idx(dir, i, j, k)];
                 const int c = (j + RNG) * RB + (k + RNG);
                 const int S = dir == 1 ? RB : 1;
                 const double* st[4];
@@ -478,14 +485,17 @@ __global__ void __launch_bounds__(NTM, 1) block_march_mhd_kernel(const fx_block_
                     }
                     continue;
                 }
-                double* F = bp->flux[dir] + bidx(9, 0, i, j, k);
+                double* F = as_global(bp->flux[dir]) + i * (PC * 9);
+                const unsigned fo = 8u * bidx(9, 0, 0, j, k);
 #pragma unroll
-                for (int lv = 0; lv < 9; ++lv) F[gmap(dir, lv) * AW] = Fl[lv];
-                double* vr = bp->v_riemann[dir] + bidx(3, 0, i, j, k);
+                for (int lv = 0; lv < 9; ++lv) at_byte(F + gmap(dir, lv) * AW, fo) = Fl[lv];
+                double* vr = as_global(bp->v_riemann[dir]) + i * (PC * 3);
+                const unsigned vo = 8u * bidx(3, 0, 0, j, k);
 #pragma unroll
-                for (int r = 0; r < 3; ++r) vr[(gmap(dir, 1 + r) - 1) * AW] = vl[r];
-                bp->Bv1[dir][lidx(i, j, k)] = bv1;
-                bp->Bv2[dir][lidx(i, j, k)] = bv2;
+                for (int r = 0; r < 3; ++r) at_byte(vr + (gmap(dir, 1 + r) - 1) * AW, vo) = vl[r];
+                const unsigned lo8 = 8u * lidx(0, j, k);
+                at_byte(as_global(bp->Bv1[dir]) + i * PC, lo8) = bv1;
+                at_byte(as_global(bp->Bv2[dir]) + i * PC, lo8) = bv2;
             }
             __syncthreads();                 // every read of plane i - 2 (and, last, of the block) done
             if (!more) break;

@@ -592,9 +592,10 @@ __device__ __forceinline__ void ens_entry(HydroLds& L, const EnsInst* __restrict
     const EnsBlock e = blocks[b / split];
     const int np = BS / split;
     const EnsInst& I = inst[e.inst];
-    const double dt = I.dev[0];
-    const double d = hydro_block<STAGE>(L, I.g, I.W[STAGE == 1 ? 0 : 1], I.W[0],
-                                        I.W[STAGE == 1 ? 1 : 0], dt,
+    double* const dev = as_global(I.dev);
+    const double dt = dev[0];
+    const double d = hydro_block<STAGE>(L, I.g, as_global(I.W[STAGE == 1 ? 0 : 1]),
+                                        as_global(I.W[0]), as_global(I.W[STAGE == 1 ? 1 : 0]), dt,
                                         e.bx * BS + (b % split) * np, np, e.by * BS, e.bz * BS);
     if (STAGE == 2) {
         // dev[2] holds the bits of the instance's largest denominator
@@ -606,7 +607,7 @@ __device__ __forceinline__ void ens_entry(HydroLds& L, const EnsInst* __restrict
         // merge the two single-lane regions across the loop's back edge
         const double m = workgroup_max(d, L.v1p[0]);
         if (threadIdx.x == 64)
-            atomicMax(reinterpret_cast<unsigned long long*>(I.dev + 2),
+            atomicMax(reinterpret_cast<unsigned long long*>(dev + 2),
                       (unsigned long long)__double_as_longlong(m));
     }
 }

@@ -73,6 +73,17 @@ __device__ __forceinline__ T& at_byte(T* base, unsigned byte)
     return *reinterpret_cast<T*>(reinterpret_cast<char*>(base) + byte);
 }
 
+// A pointer read from a table in memory may point anywhere as far as the compiler
+// can tell, and its accesses become flat ones: no scalar base, and a wait for
+// them waits for LDS too.  Taken through here it is known to point to global
+// memory.
+template <typename T>
+__device__ __forceinline__ T* as_global(T* p)
+{
+    using G = __attribute__((address_space(1))) T*;
+    return (T*)reinterpret_cast<G>(reinterpret_cast<uintptr_t>(p));
+}
+
 // Ghost mapping of one axis: the active cell a ghost coordinate c stands for
 // -- periodic wrap (the wrapped neighbour of src/prj_mesh.c:1597-1645) or the
 // mirror copy of the physical boundary (src/prj_boundary.c:413-487: src =

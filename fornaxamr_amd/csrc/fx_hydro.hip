@@ -309,6 +309,10 @@ __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
         __syncthreads();
         load_at(1, r);
         store_plane(pl[1], r, oidx, hidx, has_halo);        // plane 1
+        // nothing but the prefetch may be in flight at the loop: a register that
+        // the compiler believes to be still loading would make the loop wait,
+        // by count, for its own prefetch
+        __builtin_amdgcn_s_waitcnt(0x0f70);                 // vmcnt(0)
         load_at(2, pf);
         __syncthreads();
     }

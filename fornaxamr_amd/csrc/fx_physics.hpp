@@ -99,19 +99,56 @@ __device__ __forceinline__ double theta_limiter(double cfmax, double du, double 
 // min used for the velocity deltas (see theta_limiter)
 __device__ __forceinline__ double dmin_delta(double a, double b) { return fmin(a, b); }
 
+// sqrt(a / b) with both operations correctly rounded, for a and b in
+// [2^-300, 2^300]: Newton steps on the reciprocal and Markstein's correction of
+// the quotient, then Goldschmidt's iteration on the square root with two such
+// corrections (Markstein, IBM J. Res. Dev. 34, 1990).  The same steps as the
+// full division and square root take once they have scaled their arguments,
+// without the scaling and without the special cases: 18 instructions for 29
+// (256^3 2.13 -> 2.11 ms per step, 128^3 HLLE 254 -> 246 us).
+__device__ __forceinline__ double sqrt_ratio_mid(double a, double b)
+{
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.0), r, r);
+    r = fma(fma(-b, r, 1.0), r, r);
+    double x = a * r;
+    x = fma(fma(-b, x, a), r, x);
+    const double y = __builtin_amdgcn_rsq(x);
+    double s = x * y, h = 0.5 * y;
+    const double e = fma(-h, s, 0.5);
+    s = fma(s, e, s);
+    h = fma(h, e, h);
+    s = fma(fma(-s, s, x), h, s);
+    return fma(fma(-s, s, x), h, s);
+}
+
+// cL = sqrt(aL / rL), cR = sqrt(aR / rR).  Where all four numbers of every lane
+// are well within the range (a NaN passes the test and comes out as one), the
+// short form serves; else the full operations.  Same bits.
+__device__ __forceinline__ void sound_speeds(double aL, double rL, double aR, double rR,
+                                             double& cL, double& cR)
+{
+    const double lo = fmin(fmin(aL, rL), fmin(aR, rR)), hi = fmax(fmax(aL, rL), fmax(aR, rR));
+    if (__builtin_amdgcn_ballot_w64(lo < 0x1p-300 || hi > 0x1p300) == 0) {
+        cL = sqrt_ratio_mid(aL, rL);
+        cR = sqrt_ratio_mid(aR, rR);
+    } else {
+        cL = sqrt(aL / rL);
+        cR = sqrt(aR / rR);
+    }
+}
+
 // HLLC with the theta-limited contact speed (src/prj_riemann.c:1433-1599),
 // hydro build (6 variables).  W* are face states in the rotated frame.
 //
-// Written without branches: the reference returns F_L where 0 <= S_L, F_R
+// The reference returns F_L where 0 <= S_L, F_R
 // where S_R <= 0, and otherwise the star flux of the side the contact speed
 // selects (Toro 2009, eqs. 10.33-10.36).  Here the upwind side K is chosen
 // once -- L if 0 <= S_L, R if S_R <= 0, else by the sign of S_M -- and F_K
 // (formed from K's state by the same expressions as the reference's
 // supersonic fluxes) is taken as it is in the supersonic cases and as the base
-// of the star flux otherwise.  The star terms are evaluated in every case and
-// discarded by a select where the reference would not have formed them, so
-// every returned bit is the reference's; straight-line code lets the compiler
-// interleave the independent face solves of a cell.
+// of the star flux otherwise.  The star terms are added only where the
+// reference would have formed them, so every returned bit is the reference's.
 __device__ __forceinline__ void hllc(const double* WL, const double* WR, double pL, double pR,
                                      double gL, double gR, double du, double dv, double dw,
                                      double* flux, double* vface)
@@ -121,8 +158,8 @@ __device__ __forceinline__ void hllc(const double* WL, const double* WR, double 
     double rR = WR[RHO], uR = WR[V1], vR = WR[V2], wR = WR[V3], yR = WR[YE];
     double eL = rL * WL[EINT] + 0.5 * rL * (uL * uL + vL * vL + wL * wL);
     double eR = rR * WR[EINT] + 0.5 * rR * (uR * uR + vR * vR + wR * wR);
-    double csL = sqrt(gL * pL / rL);
-    double csR = sqrt(gR * pR / rR);
+    double csL, csR;
+    sound_speeds(gL * pL, rL, gR * pR, rR, csL, csR);
     double UL1 = rL * uL, UR1 = rR * uR;
 
     double SL = dmin(uL - csL, uR - csR);
@@ -151,22 +188,30 @@ __device__ __forceinline__ void hllc(const double* WL, const double* WR, double 
     double Fy = r * y * u;
     double rho_star = r * (S - u) / (S - SM);
     double e_over_rho = e / r + (SM - u) * (SM + p / (r * (S - u)));
-    // star fluxes formed before the selects, so that each select picks
-    // between two computed values (a conditional expression would be emitted
-    // as a branch around the star terms)
-    const double s0 = Fr + S * (rho_star - r);
-    const double s1 = Fm1 + S * (rho_star * SM - r * u);
-    const double s2 = Fm2 + S * (rho_star * v - r * v);
-    const double s3 = Fm3 + S * (rho_star * w - r * w);
-    const double s4 = Fe + S * (rho_star * e_over_rho - e);
-    const double s5 = Fy + S * (rho_star * y - r * y);
+    // The star terms are added under the lane mask: no select of 12 words per
+    // face, and none of it where a wave is supersonic throughout (128^3 278 ->
+    // 270 us per step, 112x48x80 91.8 -> 88.0).
+    const double d0 = S * (rho_star - r);
+    const double d1 = S * (rho_star * SM - r * u);
+    const double d2 = S * (rho_star * v - r * v);
+    const double d3 = S * (rho_star * w - r * w);
+    const double d4 = S * (rho_star * e_over_rho - e);
+    const double d5 = S * (rho_star * y - r * y);
     const bool sup = sup_l || sup_r;
-    flux[0] = sup ? Fr : s0;
-    flux[1] = sup ? Fm1 : s1;
-    flux[2] = sup ? Fm2 : s2;
-    flux[3] = sup ? Fm3 : s3;
-    flux[4] = sup ? Fe : s4;
-    flux[5] = sup ? Fy : s5;
+    if (!sup) {
+        Fr += d0;
+        Fm1 += d1;
+        Fm2 += d2;
+        Fm3 += d3;
+        Fe += d4;
+        Fy += d5;
+    }
+    flux[0] = Fr;
+    flux[1] = Fm1;
+    flux[2] = Fm2;
+    flux[3] = Fm3;
+    flux[4] = Fe;
+    flux[5] = Fy;
     vface[0] = sup ? u : SM;
     vface[1] = v;
     vface[2] = w;
@@ -187,8 +232,8 @@ __device__ __forceinline__ void hlle_hydro(const double* WL, const double* WR, d
     double rR = WR[RHO], uR = WR[V1], vR = WR[V2], wR = WR[V3], yR = WR[YE];
     double eL = rL * WL[EINT] + 0.5 * rL * (uL * uL + vL * vL + wL * wL);
     double eR = rR * WR[EINT] + 0.5 * rR * (uR * uR + vR * vR + wR * wR);
-    double csL = sqrt(gL * pL / rL);
-    double csR = sqrt(gR * pR / rR);
+    double csL, csR;
+    sound_speeds(gL * pL, rL, gR * pR, rR, csL, csR);
     double UL[6] = {rL, rL * uL, rL * vL, rL * wL, eL, rL * yL};
     double UR[6] = {rR, rR * uR, rR * vR, rR * wR, eR, rR * yR};
     double FL[6] = {rL * uL, rL * uL * uL + pL, rL * uL * vL, rL * uL * wL, (eL + pL) * uL,
@@ -197,21 +242,23 @@ __device__ __forceinline__ void hlle_hydro(const double* WL, const double* WR, d
                     rR * yR * uR};
     double SL = dmin(uL - csL, uR - csR);
     double SR = dmax(uL + csL, uR + csR);
-    // supersonic faces take the upwind flux; the fan terms are formed in
-    // every case and discarded there (straight-line code, same bits)
+    // supersonic faces take the upwind flux in the place of the fan's, under the
+    // lane mask (128^3 246 -> 240 us per step against selects)
     const bool sup_l = 0.0 <= SL;
     const bool sup_r = !sup_l && SR <= 0.0;
     const double inv = 1.0 / (SR - SL);
     double Uh[4];
 #pragma unroll
     for (int v = 0; v < 6; ++v) {
-        const double hll = (SR * FL[v] - SL * FR[v] + SL * SR * (UR[v] - UL[v])) * inv;
-        const double up = sup_l ? FL[v] : FR[v];
-        flux[v] = (sup_l || sup_r) ? up : hll;
+        flux[v] = (SR * FL[v] - SL * FR[v] + SL * SR * (UR[v] - UL[v])) * inv;
         if (v < 4) Uh[v] = (SR * UR[v] - SL * UL[v] + FL[v] - FR[v]) * inv;
     }
     const double vh1 = Uh[1] / Uh[0], vh2 = Uh[2] / Uh[0], vh3 = Uh[3] / Uh[0];
     const bool sup = sup_l || sup_r;
+    if (sup) {
+#pragma unroll
+        for (int v = 0; v < 6; ++v) flux[v] = sup_l ? FL[v] : FR[v];
+    }
     vface[0] = sup ? (sup_l ? uL : uR) : vh1;
     vface[1] = sup ? (sup_l ? vL : vR) : vh2;
     vface[2] = sup ? (sup_l ? wL : wR) : vh3;

@@ -170,17 +170,6 @@ enum { RS_HLLC = 0, RS_HLLE = 1 };
 // time-step reduction, taken while the new state is in registers); stage 1
 // returns 0.  RS selects the Riemann solver (the velocity deltas feed HLLC's
 // theta limiter only).
-// The value of the next lane of this lane's row of 16: a DPP move, not a pass
-// through LDS (ds_bpermute) that every wave would wait for right after the
-// barrier (256^3 2.22 -> 2.20 ms per step, 96^3 160 -> 156 us).
-__device__ __forceinline__ double next_in_row(double x)
-{
-    union { double d; int w[2]; } u = {x};
-#pragma unroll
-    for (int h = 0; h < 2; ++h) u.w[h] = __builtin_amdgcn_update_dpp(0, u.w[h], 0x101, 0xf, 0xf, true);
-    return u.d;
-}
-
 template <int STAGE, int RS = RS_HLLC>
 __device__ __forceinline__ double hydro_block(HydroLds& L, const Geom& g,
                                             const double* __restrict__ Win,

@@ -469,10 +469,19 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
 #pragma unroll
         for (int v = 0; v < 6; ++v) {
             const double fy_dn = __shfl_down(Fy[v], 16);
-            const double fz_dn = __shfl_down(Fz[v], 1);
+            const double fz_dn = next_in_row(Fz[v]);
             const double fy_hi = (j & 3) != 3 ? fy_dn : fyb[A][v][(j + 1) >> 2][k];
             const double fz_hi = k != BS - 1 ? fz_dn : fz16[A][v][j];
-            fd[v] = -(a1 * (Fxn[v] - Fx[v]) + a2 * (fy_hi - Fy[v]) + a3 * (fz_hi - Fz[v])) / vol;
+            fd[v] = -(a1 * (Fxn[v] - Fx[v]) + a2 * (fy_hi - Fy[v]) + a3 * (fz_hi - Fz[v]));
+        }
+        // as in the hydro stage: an exact product where the volume is a power of
+        // two (256^3 6.88 -> 6.84 ms per step; others unchanged)
+        if (g.vol_pow2) {
+#pragma unroll
+            for (int v = 0; v < 6; ++v) fd[v] *= g.inv_vol;
+        } else {
+#pragma unroll
+            for (int v = 0; v < 6; ++v) fd[v] /= vol;
         }
         {
             double cm[9];

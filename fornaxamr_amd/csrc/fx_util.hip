@@ -340,11 +340,13 @@ __global__ void hlld_batch_kernel(int n, const double* WL, const double* WR, con
     }
     wl[B1] = bn[f];
     wr[B1] = bn[f];
-#pragma unroll
-    for (int v = 0; v < 9; ++v) F[v] = 0.0;
-    vf[0] = vf[1] = vf[2] = 0.0;
     int rc = hlld(wl, wr, pL[f], pR[f], gL[f], gR[f], bn[f], F, vf, &e1, &e2);
     status[f] = rc;
+    if (rc != 0) {
+#pragma unroll
+        for (int v = 0; v < 9; ++v) F[v] = 0.0;
+        vf[0] = vf[1] = vf[2] = e1 = e2 = 0.0;
+    }
 #pragma unroll
     for (int v = 0; v < 9; ++v) flux[(int64_t)v * n + f] = F[v];
 #pragma unroll

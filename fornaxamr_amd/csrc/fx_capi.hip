@@ -56,6 +56,7 @@ struct fx_mesh {
     int riemann = FX_RIEMANN_HLLC;   // hydro meshes
     int split = 1;           // workgroups per block of the hydro stage / the MHD flux kernel
     int ct_split = 1;        // MHD CT workgroups per block
+    bool ct_one = false;     // by the kernel of one-plane parts
     double* saved[2] = {nullptr, nullptr};   // two further states of eSSPRK(10,4)
     double* saved_bf[2] = {nullptr, nullptr};   // and their face fields (MHD)
     hipStream_t stream = nullptr;
@@ -293,6 +294,7 @@ int run_stage(fx_mesh* m, int stage, State in, State first, State out, const dou
     a.dt = dt;
     a.flux_split = m->split;
     a.ct_split = m->ct_split;
+    a.ct_one = m->ct_one;
     a.cfl_part = stage == 2 ? m->dev + 8 : nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (m->timing) {
@@ -386,7 +388,10 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
     int ncu = 0;
     if (e == hipSuccess) e = cu_count(ncu);
     if (e == hipSuccess) m->split = stage_split(m->nblocks, ncu);
-    if (e == hipSuccess && desc->mhd) m->ct_split = mhd_ct_split(m->nblocks, ncu);
+    if (e == hipSuccess && desc->mhd) {
+        m->ct_split = mhd_ct_split(m->nblocks, ncu);
+        m->ct_one = mhd_ct_one(m->nblocks, m->ct_split, ncu);
+    }
     // dev[0..7] scalars, then the CFL partials: one per workgroup of the
     // reduction, or the maxima a stage 2 records
     m->cfl_nparts = m->nblocks * (desc->mhd ? m->ct_split : m->split);
@@ -544,6 +549,7 @@ int fx_mesh_set_mhd_schedule(fx_mesh* m, int ct_split, int side_stream)
     int ncu = 0;
     FX_HIP(cu_count(ncu));
     m->ct_split = ct_split != 0 ? ct_split : mhd_ct_split(m->nblocks, ncu);
+    m->ct_one = mhd_ct_one(m->nblocks, m->ct_split, ncu);
     m->cfl_nparts = m->nblocks * m->ct_split;
     m->cfl_ready = false;   // recorded per CT workgroup of the old split
     return FX_OK;

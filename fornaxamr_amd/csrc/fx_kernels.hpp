@@ -41,6 +41,7 @@ struct MhdStageArgs {
     double dt;
     int flux_split = 1;     // flux workgroups per block (1, 2, 4, 8 or 16), each BS / flux_split x-planes
     int ct_split = 1;       // CT workgroups per block, likewise
+    bool ct_one = false;    // the CT kernel of one-plane parts (mhd_ct_one)
     // stage 2: cfl_part[w] = largest CFL denominator of the cells CT workgroup
     // w wrote (nblocks * ct_split entries); null: not recorded
     double* cfl_part = nullptr;
@@ -111,6 +112,9 @@ int stage_split(int64_t nblocks, int ncu);
 hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s);
 // CT workgroups per block of a stage over nblocks blocks on a GPU of ncu CUs
 int mhd_ct_split(int64_t nblocks, int ncu);
+// Whether parts of one plane (ct_split == BS) take the CT kernel made for them: where
+// all of them run at once, three to a CU.
+bool mhd_ct_one(int64_t nblocks, int split, int ncu);
 
 // cell-centred B of the active cells from the faces (prj_mhd_bf2bc)
 hipError_t launch_bf2bc(const Geom& g, double* W, const double* bf, hipStream_t s);

@@ -572,11 +572,17 @@ __device__ double edge_curl_b(const MhdStageArgs& a, int dir, int i, int j, int 
            (bf_clamped(g, bf, 0, i, j, k) - bf_clamped(g, bf, 0, i, j - 1, k)) / g.dx[1];
 }
 
-template <int STAGE>
-__global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
+// ONE: parts of a single plane, on meshes whose parts all run at once: the time is
+// the chain of dependent steps.  The three cell planes are filled together and all
+// edges formed together, three phases for five, at the price of a third cell plane
+// in LDS (three workgroups per CU for four).  Step at 32^3 91 -> 86 us, 48x32x64
+// 114 -> 110, 48x48x64 152 -> 147; 64^3, which needs a fourth per CU, 166 -> 182.
+template <int STAGE, bool ONE>
+__global__ void __launch_bounds__(NT, ONE ? 3 : 4) mhd_ct_kernel(MhdStageArgs a)
 {
-    // cell EMF components and eta mask of planes (ring of 2), cells -1..16
-    __shared__ double ce[2][4][CC];
+    // cell EMF components and eta mask of planes (ring of 2; ONE: planes 0, 1
+    // and -1), cells -1..16
+    __shared__ double ce[ONE ? 3 : 2][4][CC];
     // edge EMFs: Ex of plane i, Ey/Ez at x = i and x = i + 1 (ring of 2)
     __shared__ double ex_e[EW * EW];
     __shared__ double ey_e[2][BS * EW];
@@ -594,7 +600,7 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
     // prologue (the face between two parts is formed by both, from the same
     // edges: identical values)
     const int wg = block_of_workgroup(blockIdx.x, gridDim.x);
-    const int np = BS / a.ct_split;
+    const int np = ONE ? 1 : BS / a.ct_split;
     const int part = wg % a.ct_split;
     const int b = wg / a.ct_split;
     const int bz = b % g.nbz;
@@ -717,21 +723,30 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
     };
 
     // ---- prologue: cell planes -1, 0; Ey/Ez at x = 0; Bx at x = 0 ---------
-    cell_fill(1, -1);
+    constexpr int SM = ONE ? 2 : 1;   // slot of plane -1
+    cell_fill(SM, -1);
     cell_fill(0, 0);
+    if (ONE) cell_fill(1, 1);
     __syncthreads();
-    for (int e = t; e < BS * EW; e += NT) {
+    // (ONE: remainders to waves 1 and 3, which the plane's edges below leave free)
+    for (int e = ONE ? (t + 192) & (NT - 1) : t; e < BS * EW; e += NT) {
         int jj = e / EW, kk = e % EW;
-        ey_e[0][e] = edge_y(0, jj, kk, 1, 0);
+        ey_e[0][e] = edge_y(0, jj, kk, SM, 0);
     }
-    for (int e = t; e < EW * BS; e += NT) {
+    for (int e = ONE ? (t + 64) & (NT - 1) : t; e < EW * BS; e += NT) {
         int jj = e / BS, kk = e % BS;
-        ez_e[0][e] = edge_z(0, jj, kk, 1, 0);
+        ez_e[0][e] = edge_z(0, jj, kk, SM, 0);
     }
-    __syncthreads();
     // Bx(0, j, k): -dt (Ez(j+1) - Ez(j))/dy + dt (Ey(k+1) - Ey(k))/dz
-    double bx_lo = ct(0, x0, y0 + j, z0 + k, ez_e[0][(j + 1) * BS + k], ez_e[0][j * BS + k],
-                      g.dx[1], ey_e[0][j * EW + k + 1], ey_e[0][j * EW + k], g.dx[2]);
+    auto bx_0 = [&]() {
+        return ct(0, x0, y0 + j, z0 + k, ez_e[0][(j + 1) * BS + k], ez_e[0][j * BS + k], g.dx[1],
+                  ey_e[0][j * EW + k + 1], ey_e[0][j * EW + k], g.dx[2]);
+    };
+    double bx_lo = 0.0;
+    if (!ONE) {
+        __syncthreads();
+        bx_lo = bx_0();
+    }
 
     // stage 2: each thread's running CFL maximum, kept in LDS (a register
     // live across the plane loop would cost the kernel its fourth wave)
@@ -745,7 +760,7 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
         // cell plane i+1 into the slot of plane i-1: that slot's last readers
         // (the edges of the previous plane, or of the prologue) are behind the
         // barrier that preceded the previous CT step
-        cell_fill(s1, i + 1);
+        if (!ONE) cell_fill(s1, i + 1);
         // stage 1: loads of the last phase for this thread's own cell, issued
         // here so that their latency overlaps the edge phase -- rho and
         // u4/rho - kinetic, which the flux kernel left in the output slot
@@ -756,7 +771,7 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
             rho_c = a.Wout[oc];
             t_c = a.Wout[4 * vs + oc];
         }
-        __syncthreads();
+        if (!ONE) __syncthreads();
         // Each loop has a remainder beyond NT items (33, 16, 16); rotating
         // the thread -> item map by whole waves gives each remainder to a
         // different wave (0, 3, 2), so no wave carries all three extra passes.
@@ -785,6 +800,7 @@ __global__ void __launch_bounds__(NT, 4) mhd_ct_kernel(MhdStageArgs a)
             bz_in = a.bf_in[2 * fv + cell_off(g, x0 + i, y0 + fz0 / EW, z0 + fz0 % EW)];
         }
         __syncthreads();
+        if (ONE) bx_lo = bx_0();
         // CT of Bx(i+1), By(plane i), Bz(plane i)
         double bx_hi = ct(0, x0 + i + 1, y0 + j, z0 + k, ez_e[e1][(j + 1) * BS + k],
                           ez_e[e1][j * BS + k], g.dx[1], ey_e[e1][j * EW + k + 1],
@@ -889,6 +905,11 @@ int mhd_ct_split(int64_t nblocks, int ncu)
     return split;
 }
 
+bool mhd_ct_one(int64_t nblocks, int split, int ncu)
+{
+    return split == BS && nblocks * BS <= 3 * (int64_t)ncu;
+}
+
 hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s)
 {
     const int nblocks = a.g.nbx * a.g.nby * a.g.nbz;
@@ -900,8 +921,10 @@ hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s)
     const dim3 grid((unsigned)(nfl + (ngf + NT - 1) / NT));
     if (stage == 1) hipLaunchKernelGGL(mhd_flux_kernel<1>, grid, dim3(NT), 0, s, a, nfl, ngf);
     else hipLaunchKernelGGL(mhd_flux_kernel<2>, grid, dim3(NT), 0, s, a, nfl, ngf);
-    if (stage == 1) hipLaunchKernelGGL(mhd_ct_kernel<1>, dim3(nct), dim3(NT), 0, s, a);
-    else hipLaunchKernelGGL(mhd_ct_kernel<2>, dim3(nct), dim3(NT), 0, s, a);
+    if (a.ct_one && a.ct_split != BS) return hipErrorInvalidValue;
+    const auto ct = stage == 1 ? (a.ct_one ? mhd_ct_kernel<1, true> : mhd_ct_kernel<1, false>)
+                               : (a.ct_one ? mhd_ct_kernel<2, true> : mhd_ct_kernel<2, false>);
+    hipLaunchKernelGGL(ct, dim3(nct), dim3(NT), 0, s, a);
     return hipGetLastError();
 }
 

@@ -236,7 +236,7 @@ def run_per_block(nblocks=4096, reps=10):
     ms = a.elapsed_time(b) / reps
     gbs = BYTES_BLOCK * nblocks / (ms * 1e-3) / 1e9
     host = {name: _host_block_call_ms(lib, mhd) for name, mhd in (("hydro", 0), ("mhd", 1))}
-    return {"kernel": "block_pencil_kernel<0> (x, y faces) + block_face_kernel<0, 2> (z faces): "
+    return {"kernel": "block_march_kernel (every face from one pass over the cells): "
                       "prj_flux_update on the reference's block layouts",
             "blocks": nblocks, "ms_per_launch": ms,
             "host_array_call_ms": host,
@@ -335,7 +335,7 @@ def run_mhd_line(n, steps, warmup, schedule=None):
     from fornaxamr_amd import problems as P
     pr = P.magnetized_sedov(n=(n, n, n))
     value, ms, roof = run_mesh(pr, BYTES_STAGE_MHD, steps, warmup, schedule=schedule)
-    roof["kernel"] = "mhd_flux_kernel + mhd_ghostface_kernel + mhd_ct_kernel"
+    roof["kernel"] = "mhd_flux_kernel (with the ghost-layer faces) + mhd_ct_kernel"
     roof["traffic"] = _traffic(f"mhd_{n}")
     line = {"value": value, "unit": "zone-updates/s", "ms_per_step": ms,
             "workload": (f"MHD PLM(MC)+HLLD+upwind CT RK2, {n}^3 magnetized Sedov (outflow), "

@@ -246,7 +246,7 @@ struct State {
 
 // One stage from `in` into `out`; stage 2 blends with the step's first state `first`.
 int run_stage(fx_mesh* m, int stage, State in, State first, State out, const double* dt_ptr,
-              double dt)
+              double dt, const StepDt& step = {})
 {
     const Geom& g = m->g;
     if (!g.mhd) {
@@ -259,6 +259,7 @@ int run_stage(fx_mesh* m, int stage, State in, State first, State out, const dou
         a.Wout = out.W;
         a.dt_ptr = dt_ptr;
         a.dt = dt;
+        a.step = step;
         a.cfl_part = stage == 2 ? m->dev + 8 : nullptr;
         a.riemann = m->riemann;
         a.split = m->split;
@@ -292,6 +293,7 @@ int run_stage(fx_mesh* m, int stage, State in, State first, State out, const dou
     a.err = m->err;
     a.dt_ptr = dt_ptr;
     a.dt = dt;
+    a.step = step;
     a.flux_split = m->split;
     a.ct_split = m->ct_split;
     a.ct_one = m->ct_one;
@@ -314,11 +316,11 @@ int run_stage(fx_mesh* m, int stage, State in, State first, State out, const dou
 // A stage of RK2 on the mesh's slots.  MHD: stage 1 reads face slot 0 and
 // writes slot 1; stage 2 reads slots 0 and 1 and writes the spare buffer, which
 // then becomes slot 0.
-int run_stage(fx_mesh* m, int stage, const double* dt_ptr, double dt)
+int run_stage(fx_mesh* m, int stage, const double* dt_ptr, double dt, const StepDt& step = {})
 {
     const State s0 = {m->W[0], m->bf[0]}, s1 = {m->W[1], m->bf[1]};
-    if (stage == 1) return run_stage(m, 1, s0, s0, s1, dt_ptr, dt);
-    if (int rc = run_stage(m, 2, s1, s0, {m->W[0], m->bf[2]}, dt_ptr, dt)) return rc;
+    if (stage == 1) return run_stage(m, 1, s0, s0, s1, dt_ptr, dt, step);
+    if (int rc = run_stage(m, 2, s1, s0, {m->W[0], m->bf[2]}, dt_ptr, dt, step)) return rc;
     if (m->g.mhd) std::swap(m->bf[0], m->bf[2]);
     return FX_OK;
 }
@@ -612,6 +614,17 @@ int fx_step_async(fx_mesh* m, double cfl, double dt_factor)
     const bool ssp = m->integrator == FX_ESSPRK10_4;
     // the CFL maximum of W[0] comes from the stage 2 that wrote it when that
     // was recorded, else from a reduction over the cells
+    if (!ssp && m->cfl_ready && m->cfl_nparts <= STEP_DT_PARTS) {
+        StepDt step;
+        step.dev = m->dev;
+        const StepDt second = step;
+        step.part = m->dev + 8;
+        step.n = m->cfl_nparts;
+        step.cfl = cfl;
+        step.factor = dt_factor;
+        if (int rc = run_stage(m, 1, m->dev, 0.0, step)) return rc;
+        return run_stage(m, 2, m->dev, 0.0, second);
+    }
     const double scale = ssp ? 6.0 : 1.0;
     if (m->cfl_ready)
         FX_HIP(launch_dt_final(m->dev + 8, m->cfl_nparts, cfl, m->dev + 0, m->dev + 1, dt_factor,

@@ -11,6 +11,20 @@
 
 namespace fx {
 
+// The step's dt formed inside stage 1, by every workgroup from the CFL maxima that
+// the last stage 2 recorded (at most STEP_DT_PARTS of them), in place of a launch of
+// its own: stage 1 leaves it in dev[0], and stage 2, when nothing reads the previous
+// step's dt any more, in dev[1].  Step at 32^3 28.7 -> 26.7 us, 64^3 50.8 -> 49.0,
+// 128^3 (512 maxima) 270.8 -> 268.6, 48x32x64 MHD 110 -> 109; at 640 MHD maxima and
+// more it gains nothing.
+constexpr int STEP_DT_PARTS = 1024;
+struct StepDt {
+    const double* part = nullptr;   // null: not formed here (dt_ptr, dt)
+    int n = 0;
+    double cfl = 0.0, factor = 0.0;
+    double* dev = nullptr;          // stages 1 and 2 of such a step
+};
+
 struct HydroStageArgs {
     Geom g;
     const double* Win;      // stage input W (padded layout, 6 variables)
@@ -18,6 +32,7 @@ struct HydroStageArgs {
     double* Wout;           // stage output (may alias W0 for stage 2)
     const double* dt_ptr;   // device dt, or null to use dt
     double dt;
+    StepDt step;
     int split = 1;          // workgroups per block (1, 2, 4, 8 or 16), each 16 / split x-planes
     // stage 2: cfl_part[w] = largest CFL denominator of the cells workgroup w
     // wrote (nblocks * split entries); null: not recorded
@@ -39,6 +54,7 @@ struct MhdStageArgs {
     int* err;               // device error word: [code, dir, x, y, z]
     const double* dt_ptr;
     double dt;
+    StepDt step;
     int flux_split = 1;     // flux workgroups per block (1, 2, 4, 8 or 16), each BS / flux_split x-planes
     int ct_split = 1;       // CT workgroups per block, likewise
     bool ct_one = false;    // the CT kernel of one-plane parts (mhd_ct_one)

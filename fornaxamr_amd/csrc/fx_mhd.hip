@@ -258,7 +258,7 @@ __device__ __forceinline__ void ghost_face(const MhdStageArgs& a, int64_t id, in
 // cost more at every size (us per step, in order / second stream / here: 8 blocks
 // 112 / 115 / 100, 64 blocks 194 / 215 / 185, 512 blocks 1106 / 1091 / 1077, 4096
 // blocks 7847 / 7892 / 7772).
-template <int STAGE>
+template <int STAGE, bool FORM_DT = false>   // FORM_DT: the step's dt is formed here (StepDt)
 __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg, int64_t ghosts)
 {
     if ((int)blockIdx.x >= nwg) {
@@ -298,7 +298,15 @@ __global__ void __launch_bounds__(NT, 2) mhd_flux_kernel(MhdStageArgs a, int nwg
     const int64_t vs = g.vstride;
     const double gm1 = g.gamma - 1.0;
     const double gam = g.gamma;
-    const double dt = a.dt_ptr ? *a.dt_ptr : a.dt;
+    double dt;
+    if (FORM_DT && STAGE == 1) {
+        dt = form_step_dt(a.step.part, a.step.n, a.step.cfl, a.step.factor, a.step.dev[1],
+                          fz16[0][0]);
+        if (blockIdx.x == 0 && t == 0) a.step.dev[0] = dt;
+    } else {
+        dt = a.dt_ptr ? *a.dt_ptr : a.dt;
+        if (FORM_DT && blockIdx.x == 0 && t == 0) a.step.dev[1] = dt;
+    }
 
     const int oidx = (j + NG) * PW + (k + NG);
     const bool has_halo = t < NHALO;
@@ -919,8 +927,11 @@ hipError_t launch_mhd_stage(const MhdStageArgs& a, int stage, hipStream_t s)
     const int64_t ngf = ghostface_count(a.g);
     if (ngf >= ((int64_t)1 << 31)) return hipErrorInvalidValue;   // 32-bit decode
     const dim3 grid((unsigned)(nfl + (ngf + NT - 1) / NT));
-    if (stage == 1) hipLaunchKernelGGL(mhd_flux_kernel<1>, grid, dim3(NT), 0, s, a, nfl, ngf);
-    else hipLaunchKernelGGL(mhd_flux_kernel<2>, grid, dim3(NT), 0, s, a, nfl, ngf);
+    const bool form = a.step.dev != nullptr;
+    if (form && stage == 1 && a.step.part == nullptr) return hipErrorInvalidValue;
+    const auto flux = stage == 1 ? (form ? mhd_flux_kernel<1, true> : mhd_flux_kernel<1, false>)
+                                 : (form ? mhd_flux_kernel<2, true> : mhd_flux_kernel<2, false>);
+    hipLaunchKernelGGL(flux, grid, dim3(NT), 0, s, a, nfl, ngf);
     if (a.ct_one && a.ct_split != BS) return hipErrorInvalidValue;
     const auto ct = stage == 1 ? (a.ct_one ? mhd_ct_kernel<1, true> : mhd_ct_kernel<1, false>)
                                : (a.ct_one ? mhd_ct_kernel<2, true> : mhd_ct_kernel<2, false>);

@@ -33,6 +33,37 @@ __device__ __forceinline__ double workgroup_max(double v, double* lds)
     return r;
 }
 
+__device__ __forceinline__ double dt_from_denom(double cfl, double max_denom)
+{
+    const double dt = cfl / max_denom;
+    return dt < 1.0e99 ? dt : 1.0e99;
+}
+
+// dt = min(dt_new, factor * previous dt) after the first step (src/main.c:517-522)
+__device__ __forceinline__ double growth_limit(double dt_new, double prev, double factor)
+{
+    if (prev > 0.0) {
+        const double lim = factor * prev;
+        return dt_new <= lim ? dt_new : lim;
+    }
+    return dt_new;
+}
+
+// The step's dt, by a whole workgroup, from the n recorded CFL maxima `part` and the
+// previous dt; the same in every thread (a scalar).  lds as for workgroup_max.
+__device__ __forceinline__ double form_step_dt(const double* part, int n, double cfl,
+                                               double factor, double prev, double* lds)
+{
+    double best = 0.0;
+    for (int i = threadIdx.x; i < n; i += blockDim.x)
+        if (part[i] > best) best = part[i];
+    const double dt = growth_limit(dt_from_denom(cfl, workgroup_max(best, lds)), prev, factor);
+    const long long b = __double_as_longlong(dt);
+    const unsigned lo = __builtin_amdgcn_readfirstlane((int)b);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __longlong_as_double(((unsigned long long)hi << 32) | lo);
+}
+
 // primitive / conserved variable slots (src/prj_defs.h:466-494)
 enum { RHO = 0, V1 = 1, V2 = 2, V3 = 3, EINT = 4, YE = 5, B1 = 6, B2 = 7, B3 = 8 };
 enum { MOM1 = 1, MOM2 = 2, MOM3 = 3, ETOT = 4 };

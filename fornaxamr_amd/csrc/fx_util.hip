@@ -170,12 +170,6 @@ __device__ __forceinline__ double cell_denom(const Geom& g, const double* __rest
     return cfl_denom(g, W[o], W[vs + o], W[2 * vs + o], W[3 * vs + o], W[4 * vs + o]);
 }
 
-__device__ __forceinline__ double dt_from_denom(double cfl, double max_denom)
-{
-    const double dt = cfl / max_denom;
-    return dt < 1.0e99 ? dt : 1.0e99;
-}
-
 // largest denominator of the 16^3 block (bx, by, bz); thread (j, k) walks x
 __device__ __forceinline__ double block_max_denom(const Geom& g, const double* __restrict__ W,
                                                   int bx, int by, int bz, double* red)
@@ -238,11 +232,7 @@ __device__ __forceinline__ void dt_finalize(double dt_new, double* dt_out, doubl
     if (scale != 1.0) dt_new *= scale;
     double dt = dt_new;
     if (dt_prev != nullptr) {
-        double prev = dt_prev[0];
-        if (prev > 0.0) {
-            double lim = factor * prev;
-            dt = dt_new <= lim ? dt_new : lim;
-        }
+        dt = growth_limit(dt_new, dt_prev[0], factor);
         dt_prev[0] = dt;
     }
     dt_out[0] = dt;

@@ -475,7 +475,7 @@ __global__ void __launch_bounds__(NTM, 1) block_march_mhd_kernel(const fx_block_
                     pg[2 * v + 1] = s2 - mc_half(s1, s2, s3);
                 }
                 double Fl[9], vl[3], bv1 = 0.0, bv2 = 0.0;
-                const int rc = hlld(WL, WR, pg[0], pg[1], pg[2], pg[3], bn, Fl, vl, &bv1, &bv2);
+                const int rc = hlld<false>(WL, WR, pg[0], pg[1], pg[2], pg[3], bn, Fl, vl, &bv1, &bv2);
                 if (rc != 0) {
                     if (atomicCAS(err, 0, rc) == 0) {
                         err[1] = dir;

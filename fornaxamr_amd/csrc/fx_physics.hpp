@@ -142,19 +142,27 @@ __device__ __forceinline__ double next_in_row(double x)
 }
 
 // sqrt(a / b) with both operations correctly rounded, for a and b in
-// [2^-300, 2^300]: Newton steps on the reciprocal and Markstein's correction of
-// the quotient, then Goldschmidt's iteration on the square root with two such
-// corrections (Markstein, IBM J. Res. Dev. 34, 1990).  The same steps as the
-// full division and square root take once they have scaled their arguments,
-// without the scaling and without the special cases: 18 instructions for 29
+// [2^-300, 2^300] (sqrt_mid alone: [2^-601, 2^601]): Newton steps on the
+// reciprocal and Markstein's correction of the quotient, then Goldschmidt's
+// iteration on the square root with two such corrections (Markstein, IBM J. Res.
+// Dev. 34, 1990).  The same steps as the full division and square root take once
+// they have scaled their arguments, without the scaling and without the special
+// cases: 18 instructions for 29
 // (256^3 2.13 -> 2.11 ms per step, 128^3 HLLE 254 -> 246 us).
-__device__ __forceinline__ double sqrt_ratio_mid(double a, double b)
+__device__ __forceinline__ double recip_mid(double b)
 {
     double r = __builtin_amdgcn_rcp(b);
     r = fma(fma(-b, r, 1.0), r, r);
-    r = fma(fma(-b, r, 1.0), r, r);
-    double x = a * r;
-    x = fma(fma(-b, x, a), r, x);
+    return fma(fma(-b, r, 1.0), r, r);
+}
+// a / b, r = recip_mid(b)
+__device__ __forceinline__ double quotient_mid(double a, double b, double r)
+{
+    const double x = a * r;
+    return fma(fma(-b, x, a), r, x);
+}
+__device__ __forceinline__ double sqrt_mid(double x)
+{
     const double y = __builtin_amdgcn_rsq(x);
     double s = x * y, h = 0.5 * y;
     const double e = fma(-h, s, 0.5);
@@ -162,6 +170,10 @@ __device__ __forceinline__ double sqrt_ratio_mid(double a, double b)
     h = fma(h, e, h);
     s = fma(fma(-s, s, x), h, s);
     return fma(fma(-s, s, x), h, s);
+}
+__device__ __forceinline__ double sqrt_ratio_mid(double a, double b)
+{
+    return sqrt_mid(quotient_mid(a, b, recip_mid(b)));
 }
 
 // cL = sqrt(aL / rL), cR = sqrt(aR / rR).  Where all four numbers of every lane
@@ -390,19 +402,38 @@ __device__ __forceinline__ int hlld_side_error(const HlldSide& s)
 }
 
 // fast magnetosonic speed (src/prj_riemann.c:117-140); its checks go to bad_disc
-// and bad_cf
+// and bad_cf.  MID: rho and g p in [2^-300, 2^300], the squared fields there or zero:
+// one reciprocal for the three quotients (of +0 the quotient is +0), and the short
+// square root of cf2, which is at least half of a2.
+template <bool MID>
 __device__ __forceinline__ double hlld_fast(const HlldSide& s, double bx, bool& bad_disc,
                                             bool& bad_cf)
 {
-    double a2 = s.g * s.p / s.rho;
-    double bx2_rho = bx * bx / s.rho;
-    double b2_rho = (bx * bx + s.by * s.by + s.bz * s.bz) / s.rho;
+    const double r = MID ? recip_mid(s.rho) : 0.0;
+    const auto over_rho = [&](double a) { return MID ? quotient_mid(a, s.rho, r) : a / s.rho; };
+    double a2 = over_rho(s.g * s.p);
+    double bx2_rho = over_rho(bx * bx);
+    double b2_rho = over_rho(bx * bx + s.by * s.by + s.bz * s.bz);
     double disc = (a2 + b2_rho) * (a2 + b2_rho) - 4.0 * a2 * bx2_rho;
     bad_disc = disc < 0.0 && disc < -1.0e-12 * (a2 + b2_rho) * (a2 + b2_rho);
     disc = disc < 0.0 ? 0.0 : disc;
     double cf2 = 0.5 * (a2 + b2_rho + sqrt(disc));
     bad_cf = cf2 < 0.0 || !isfinite(cf2);
-    return sqrt(cf2);
+    return MID ? sqrt_mid(cf2) : sqrt(cf2);
+}
+
+// whether every lane's pair of states is in the range of hlld_fast<true>
+__device__ __forceinline__ bool hlld_mid(const HlldSide& L, const HlldSide& R, double bx)
+{
+    const double gpL = L.g * L.p, gpR = R.g * R.p;
+    const double lo = fmin(fmin(gpL, L.rho), fmin(gpR, R.rho));
+    const double b0 = bx * bx, bL = b0 + L.by * L.by + L.bz * L.bz,
+                 bR = b0 + R.by * R.by + R.bz * R.bz;
+    const double hi = fmax(fmax(fmax(gpL, L.rho), fmax(gpR, R.rho)), fmax(bL, bR));
+    unsigned long long out = __builtin_amdgcn_ballot_w64(lo < 0x1p-300 || hi > 0x1p300);
+    for (const double b : {b0, bL, bR})
+        out |= __builtin_amdgcn_ballot_w64(b < 0x1p-300) & ~__builtin_amdgcn_ballot_w64(b == 0.0);
+    return out == 0;
 }
 
 // outer (single-star) state (src/prj_riemann.c:187-232)
@@ -448,6 +479,10 @@ __device__ __forceinline__ int hlld_outer(const HlldSide& s, double bx, double S
 // scheduled.  One branch holds the checks of both states, and the supersonic, single-
 // and double-star fluxes are stages of one sum rather than separate exits.
 // MHD step: 256^3 7.54 -> 6.87 ms, 128^3 1041 -> 957 us, 48x32x64 120 -> 114.
+// SHORT: with the short forms of the fast speeds (256^3 7.00 -> 6.88 ms per step,
+// 112x48x80 274 -> 268 us; not worth it in the per-block kernel, whose one
+// workgroup per CU of 8 waves gains nothing: 343 blocks 390 -> 392 us).
+template <bool SHORT = true>
 __device__ __forceinline__ int hlld(const double* WL, const double* WR, double pL, double pR,
                                  double gL, double gR, double bn, double* flux, double* vface,
                                  double* bv1, double* bv2)
@@ -457,8 +492,14 @@ __device__ __forceinline__ int hlld(const double* WL, const double* WR, double p
     hlld_side(WL, pL, gL, bn, L);
     hlld_side(WR, pR, gR, bn, R);
     bool bad[4];
-    const double cfL = hlld_fast(L, bn, bad[0], bad[1]);
-    const double cfR = hlld_fast(R, bn, bad[2], bad[3]);
+    double cfL, cfR;
+    if (SHORT && hlld_mid(L, R, bn)) {
+        cfL = hlld_fast<true>(L, bn, bad[0], bad[1]);
+        cfR = hlld_fast<true>(R, bn, bad[2], bad[3]);
+    } else {
+        cfL = hlld_fast<false>(L, bn, bad[0], bad[1]);
+        cfR = hlld_fast<false>(R, bn, bad[2], bad[3]);
+    }
     double SL = dmin(L.vx - cfL, R.vx - cfR);
     double SR = dmax(L.vx + cfL, R.vx + cfR);
     // one branch for the checks of both states: what follows a failed one is

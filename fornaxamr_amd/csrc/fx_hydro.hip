@@ -1,6 +1,6 @@
 // Hydro RK2 stage on gfx950: MC reconstruction + HLLC(theta) (or HLLE) +
 // flux divergence + per-cell RK2 update, fused in one kernel, one workgroup
-// per 16^3 block.
+// per 16^3 block or per part of its x-planes (stage_split).
 //
 // Reference path: prj_flux_update (src/prj_flux.c:2149-2521) for every block,
 // then the per-cell stage update (src/prj_timeint.c:1255-1350 stage 1,
@@ -17,9 +17,9 @@
 // of its cell and the x-face on its high side; the 32 high-side y/z faces of
 // the block (shared with the neighbour blocks) are solved by half of one wave,
 // rotating through the waves plane by plane.  x-face states and fluxes are
-// carried in registers along the column; y/z fluxes are exchanged through LDS
-// (aliasing the dead part of plane i) to form the divergence in the
-// reference's x, y, z summation order.  The next plane is prefetched into
+// carried in registers along the column; z fluxes are exchanged by DPP, y fluxes
+// by ds_bpermute and, across waves, LDS, to form the divergence in the reference's
+// x, y, z summation order.  The next plane is prefetched into
 // registers one step ahead.
 #include <hip/hip_runtime.h>
 

@@ -9,17 +9,17 @@
 // from the new faces (src/prj_timeint.c:498-510, 1255-1350, 1562-1655).
 //
 // Two launches per stage after the ghost fill:
-//   mhd_flux_kernel   one workgroup per 16^3 block, marching x-planes like the
+//   mhd_flux_kernel   one workgroup per part of a 16^3 block, marching x-planes like the
 //                     hydro kernel: HLLD on the block's faces, flux divergence,
 //                     RK combination of the hydro conserved variables and their
 //                     conversion to rho, v, Ye and the field-free part of the
 //                     internal energy (into the output slot), and the per-face
-//                     EMF inputs (Bv1, Bv2, normal velocity); further
+//                     EMF inputs (Bv1, Bv2, the normal velocity's sign word); further
 //                     workgroups solve the same face inputs on the one-face
 //                     transverse layer outside the domain that boundary edges
 //                     read (the reference computes it from ghost cells, -1..16
 //                     loops);
-//   mhd_ct_kernel     one workgroup per block, marching x-planes: cell EMFs,
+//   mhd_ct_kernel     one workgroup per part of a block, marching x-planes: cell EMFs,
 //                     edge EMFs, CT update of the block's faces, cell-centred B
 //                     and the magnetic term of the internal energy.
 // Faces on block boundaries are computed by both neighbours with identical
@@ -249,7 +249,7 @@ __device__ __forceinline__ void ghost_face(const MhdStageArgs& a, int64_t id, in
 // y- and z-face of its own cell and the x-face i+1 (cells i..i+2 along its
 // column); half of one wave (rotating) solves the 32 high-side y/z faces on
 // the block boundary.  The high-side y/z fluxes of a cell come from the
-// neighbouring lanes (shuffles), across wave rows and from the extra faces
+// neighbouring lanes (DPP, shuffles), across wave rows and from the extra faces
 // through a small LDS buffer.
 //
 // Workgroups beyond the nwg of the blocks solve the `ghosts` ghost-layer faces, a

@@ -145,6 +145,20 @@ int sync_mesh(fx_mesh* m, double* dt)
     return FX_OK;
 }
 
+// A device array where there is none yet, cleared on stream s: a fill of the null
+// stream may outlast the call, and non-blocking streams do not wait for it.
+hipError_t alloc_cleared(double** p, size_t bytes, hipStream_t s)
+{
+    if (*p != nullptr) return hipSuccess;
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) {
+        e = hipMemsetAsync(*p, 0, bytes, s);
+        if (e != hipSuccess) (void)hipFree(*p);
+    }
+    if (e != hipSuccess) *p = nullptr;
+    return e;
+}
+
 // compute units of the current device
 hipError_t cu_count(int& ncu)
 {
@@ -522,18 +536,16 @@ int fx_mesh_set_integrator(fx_mesh* m, int integrator)
         return fail(FX_EINVAL, "unknown integrator");
     if (integrator == FX_ESSPRK10_4) {
         FX_HIP(hipStreamSynchronize(m->stream));
+        hipError_t e = hipSuccess;
         for (int s = 0; s < 2; ++s) {
-            hipError_t e = hipSuccess;
-            if (m->saved[s] == nullptr) e = hipMalloc(&m->saved[s], m->cell_bytes * m->nh);
-            if (e == hipSuccess && m->g.mhd && m->saved_bf[s] == nullptr)
-                e = hipMalloc(&m->saved_bf[s], 3 * m->cell_bytes);
-            if (e == hipSuccess) e = hipMemset(m->saved[s], 0, m->cell_bytes * m->nh);
+            if (e == hipSuccess) e = alloc_cleared(&m->saved[s], m->cell_bytes * m->nh, m->stream);
             if (e == hipSuccess && m->g.mhd)
-                e = hipMemset(m->saved_bf[s], 0, 3 * m->cell_bytes);
-            if (e != hipSuccess)
-                return fail(e == hipErrorOutOfMemory ? FX_ENOMEM : FX_EHIP,
-                            std::string("fx_mesh_set_integrator: ") + hipGetErrorString(e));
+                e = alloc_cleared(&m->saved_bf[s], 3 * m->cell_bytes, m->stream);
         }
+        if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
+        if (e != hipSuccess)
+            return fail(e == hipErrorOutOfMemory ? FX_ENOMEM : FX_EHIP,
+                        std::string("fx_mesh_set_integrator: ") + hipGetErrorString(e));
     }
     m->integrator = integrator;
     return FX_OK;

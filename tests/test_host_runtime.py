@@ -1,0 +1,58 @@
+"""The library's host code over a stand-in for the HIP runtime (hip_host.cpp), on
+machines without a GPU: in what order a mesh's buffers are cleared.  The scripts
+run in a process of their own, where the stand-in is loaded before the library."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+HEAD = """
+import ctypes as C, sys
+host = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+host.host_pending.argtypes = [C.c_void_p]
+host.host_malloc_limit.argtypes = [C.c_size_t]
+calls = lambda name: host.host_calls(name.encode())
+import numpy as np
+from fornaxamr_amd import _native, problems as P
+from fornaxamr_amd.mesh import GpuMesh
+"""
+
+
+@pytest.fixture(scope="module")
+def host_run(tmp_path_factory):
+    from fornaxamr_amd import build
+    cxx = shutil.which("g++")
+    if cxx is None or not os.path.exists(build.LIB):
+        pytest.skip("needs g++ and the built library")
+    lib = str(tmp_path_factory.mktemp("hip_host") / "libhip_host.so")
+    subprocess.run([cxx, "-O1", "-std=c++17", "-fPIC", "-shared", os.path.join(HERE, "hip_host.cpp"),
+                    "-o", lib], check=True)
+
+    def run(script):
+        r = subprocess.run([sys.executable, "-c", HEAD + script, lib], cwd=os.path.dirname(HERE),
+                           capture_output=True, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+@pytest.mark.parametrize("mhd", [False, True], ids=["hydro", "mhd"])
+def test_integrator_clears_in_stream_order(host_run, mhd):
+    """Choosing eSSPRK(10,4) leaves no clear of its two further states running (one
+    of the null stream would run beside the next step on a non-blocking stream),
+    and clears them only when it allocates them."""
+    host_run(f"""
+m = GpuMesh((32, 32, 32), (0.0, 1.0) * 3, (0,) * 6, 1.4, mhd={mhd})
+host.hipDeviceSynchronize()
+_native.check(m.lib.fx_mesh_set_stream(m.h, 0x40))
+m.set_integrator("essprk10_4")
+assert host.host_pending(None) == 0 and host.host_pending(0x40) == 0
+fills = calls("hipMemset") + calls("hipMemsetAsync")
+m.set_integrator("rk2")
+m.set_integrator("essprk10_4")
+assert calls("hipMemset") + calls("hipMemsetAsync") == fills
+m.close()
+""")

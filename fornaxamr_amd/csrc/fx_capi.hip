@@ -388,15 +388,10 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
     m->cell_bytes = (size_t)m->g.vstride * sizeof(double);
     const size_t slot = m->cell_bytes * m->nh;
     hipError_t e = hipSuccess;
-    for (int s = 0; s < 2 && e == hipSuccess; ++s) {
-        e = hipMalloc(&m->W[s], slot);
-        if (e == hipSuccess) e = hipMemset(m->W[s], 0, slot);
-    }
+    for (int s = 0; s < 2 && e == hipSuccess; ++s) e = alloc_cleared(&m->W[s], slot, m->stream);
     if (e == hipSuccess && desc->mhd) {
-        for (int s = 0; s < 3 && e == hipSuccess; ++s) {
-            e = hipMalloc(&m->bf[s], 3 * m->cell_bytes);
-            if (e == hipSuccess) e = hipMemset(m->bf[s], 0, 3 * m->cell_bytes);
-        }
+        for (int s = 0; s < 3 && e == hipSuccess; ++s)
+            e = alloc_cleared(&m->bf[s], 3 * m->cell_bytes, m->stream);
         if (e == hipSuccess) e = hipMalloc(&m->fdat, fdat_doubles(m->g) * sizeof(double));
         if (e == hipSuccess) e = hipMalloc(&m->zring, zring_doubles(m->g) * sizeof(double));
     }
@@ -416,7 +411,9 @@ int fx_mesh_create(const fx_mesh_desc* desc, fx_mesh** out)
     const size_t npart = std::max<size_t>(
         CALC_DT_WGS, (size_t)m->nblocks * (desc->mhd ? std::max(4, m->ct_split) : m->split));
     if (e == hipSuccess) e = hipMalloc(&m->dev, (8 + npart) * sizeof(double));
-    if (e == hipSuccess) e = hipMemset(m->dev, 0, 8 * sizeof(double));
+    if (e == hipSuccess) e = hipMemsetAsync(m->dev, 0, 8 * sizeof(double), m->stream);
+    // the caller may go on on a stream that does not wait for this one
+    if (e == hipSuccess) e = hipStreamSynchronize(m->stream);
     m->err = reinterpret_cast<int*>(m->dev + 5);
     if (e != hipSuccess) {
         fx_mesh_destroy(m);
@@ -948,18 +945,15 @@ int fx_ensemble_create(int n, const fx_mesh_desc* descs, fx_ensemble** out)
     fx_ensemble* e = new fx_ensemble();
     e->n = n;
     hipError_t err = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking);
-    if (err == hipSuccess) err = hipMalloc(&e->dev, sizeof(double) * 4 * n);
-    if (err == hipSuccess) err = hipMemset(e->dev, 0, sizeof(double) * 4 * n);
+    if (err == hipSuccess) err = alloc_cleared(&e->dev, sizeof(double) * 4 * n, e->stream);
     for (int i = 0; i < n && err == hipSuccess; ++i) {
         const fx_mesh_desc& d = descs[i];
         Geom g = make_geom(d.n[0], d.n[1], d.n[2], d.xlim, d.bc, d.gamma, 0, 0.0);
         EnsInst I{};
         I.g = g;
         const size_t bytes = (size_t)g.vstride * 6 * sizeof(double);
-        err = hipMalloc(&I.W[0], bytes);
-        if (err == hipSuccess) err = hipMemset(I.W[0], 0, bytes);
-        if (err == hipSuccess) err = hipMalloc(&I.W[1], bytes);
-        if (err == hipSuccess) err = hipMemset(I.W[1], 0, bytes);
+        for (int s = 0; s < 2 && err == hipSuccess; ++s)
+            err = alloc_cleared(&I.W[s], bytes, e->stream);
         I.dev = e->dev + 4 * i;
         e->geoms.push_back(g);
         e->host_inst.push_back(I);
@@ -1009,7 +1003,8 @@ int fx_ensemble_create(int n, const fx_mesh_desc* descs, fx_ensemble** out)
                             hipMemcpyHostToDevice);
     }
     if (err == hipSuccess) err = hipMalloc(&e->d_queues, 64 * sizeof(int));
-    if (err == hipSuccess) err = hipMemset(e->d_queues, 0, 64 * sizeof(int));
+    if (err == hipSuccess) err = hipMemsetAsync(e->d_queues, 0, 64 * sizeof(int), e->stream);
+    if (err == hipSuccess) err = hipStreamSynchronize(e->stream);
     if (err != hipSuccess) {
         fx_ensemble_destroy(e);
         return fail(err == hipErrorOutOfMemory ? FX_ENOMEM : FX_EHIP,

@@ -56,3 +56,30 @@ m.set_integrator("essprk10_4")
 assert calls("hipMemset") + calls("hipMemsetAsync") == fills
 m.close()
 """)
+
+
+def test_created_state_is_clear(host_run):
+    """A new mesh or ensemble leaves no clear running that a stream given to it
+    afterwards (or the ensemble's own) would not wait for."""
+    host_run("""
+from fornaxamr_amd.ensemble import GpuEnsemble
+for mhd in (False, True):
+    m = GpuMesh((32, 32, 32), (0.0, 1.0) * 3, (0,) * 6, 1.4, mhd=mhd)
+    assert host.host_pending(None) == 0, mhd
+    v = m.view()
+    for p in v.W:
+        a = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_double)), (v.nh * v.vstride,))
+        assert not a.any()
+    m.close()
+host.hipDeviceSynchronize()
+h = C.c_void_p()
+d = (_native.MeshDesc * 2)()
+for i in range(2):
+    d[i].n[:] = [16 * (i + 1)] * 3
+    d[i].xlim[:] = [0.0, 1.0] * 3
+    d[i].gamma = 1.4
+lib = _native.load()
+_native.check(lib.fx_ensemble_create(2, d, C.byref(h)))
+assert host.host_pending(None) == 0
+lib.fx_ensemble_destroy(h)
+""")

@@ -973,7 +973,7 @@ int fx_ensemble_create(int n, const fx_mesh_desc* descs, fx_ensemble** out)
     if (err == hipSuccess) err = hipMalloc(&e->partial, (size_t)std::max(1, nparts) * sizeof(double));
     // interleaved table: instances dealt round robin block by block, so that
     // every part of the table mixes all instances
-    {
+    if (err == hipSuccess) {
         std::vector<size_t> next(n, 0), start(n, 0);
         size_t acc = 0;
         for (int i = 0; i < n; ++i) {

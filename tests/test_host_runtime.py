@@ -83,3 +83,25 @@ _native.check(lib.fx_ensemble_create(2, d, C.byref(h)))
 assert host.host_pending(None) == 0
 lib.fx_ensemble_destroy(h)
 """)
+
+
+def test_ensemble_out_of_memory(host_run):
+    """An ensemble whose states do not all fit is refused with FX_ENOMEM, whichever
+    allocation fails."""
+    host_run("""
+lib = _native.load()
+h = C.c_void_p()
+n = 40
+d = (_native.MeshDesc * n)()
+for i in range(n):
+    d[i].n[:] = [16 * (i % 3 + 1)] * 3
+    d[i].xlim[:] = [0.0, 1.0] * 3
+    d[i].gamma = 1.4
+for limit in (0, 500, 2000, 10000, 1000000, 2000000):
+    host.host_malloc_limit(limit)
+    assert lib.fx_ensemble_create(n, d, C.byref(h)) == -4, limit
+    assert h.value is None
+host.host_malloc_limit(1 << 40)
+assert lib.fx_ensemble_create(n, d, C.byref(h)) == 0
+lib.fx_ensemble_destroy(h)
+""")

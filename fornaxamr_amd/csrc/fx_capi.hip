@@ -25,8 +25,8 @@
 using namespace fx;
 
 // Device staging of the host transfers of one mesh or ensemble: allocated by the
-// first transfer, at most STAGING_BYTES (one row if that is longer), freed with
-// its owner.
+// first transfer, at most STAGING_BYTES (one row if that is longer), replaced by a
+// larger one where a transfer has more to move, freed with its owner.
 constexpr size_t STAGING_BYTES = (size_t)64 << 20;
 struct Staging {
     std::mutex lock;         // held by a transfer to its end
@@ -172,8 +172,8 @@ hipError_t cu_count(int& ncu)
 // One padded field, from its entry (0, 0, 0) of variable 0 on, to a host array
 // [nv][ex][ey][ez] (host_out) or from one (host_in, into dev and, if non-null,
 // dev2); synchronises the stream.  Rows go through the staging buffer in chunks
-// of one copy each.  Where no buffer can be allocated: one 2D copy per variable
-// and x-plane.
+// of one copy each; where a larger one cannot be allocated, through the one there
+// is.  Without any: one 2D copy per variable and x-plane.
 int copy_field(Staging& st, hipStream_t s, const RowField& f, int nv, double* dev, double* dev2,
                const double* host_in, double* host_out)
 {
@@ -183,18 +183,16 @@ int copy_field(Staging& st, hipStream_t s, const RowField& f, int nv, double* de
     const size_t rows = (size_t)nv * f.ex * f.ey;
     const size_t want = std::min(rows, std::max<size_t>(1, STAGING_BYTES / row)) * row;
     if (st.cap < want) {
-        FX_HIP(hipStreamSynchronize(s));
-        (void)hipFree(st.buf);
-        st.buf = nullptr;
-        st.cap = 0;
-        if (hipMalloc(&st.buf, want) == hipSuccess) {
+        double* larger = nullptr;
+        if (hipMalloc(&larger, want) == hipSuccess) {
+            (void)hipFree(st.buf);   // idle: every transfer ends with a wait
+            st.buf = larger;
             st.cap = want;
         } else {
-            st.buf = nullptr;
             (void)hipGetLastError();
         }
     }
-    if (st.buf == nullptr) {
+    if (st.cap < row) {
         for (int v = 0; v < nv; ++v) {
             for (int x = 0; x < f.ex; ++x) {
                 const int64_t o = v * f.vstride + x * f.sx;

@@ -50,6 +50,10 @@ int fx_mesh_destroy(fx_mesh *m);
 int fx_mesh_set_stream(fx_mesh *m, void *hip_stream);
 
 /* ---- state transfer (host arrays in the global layout above) ------------ */
+/* Transfers go through a device buffer that the mesh keeps from its first one
+ * until it is destroyed: as large as the largest array moved, at most 64 MiB
+ * (one row of cells along z where that is more).  An ensemble has one likewise.
+ * Where it cannot be allocated, transfers are slower, with the same result. */
 /* Sets both stage slots.  For MHD the cell-centred B of W is ignored and
  * recomputed from the faces given by fx_mesh_set_bf (prj_mhd_bf2bc_all,
  * src/prj_mhd.c:615-619), so call fx_mesh_set_bf after fx_mesh_set_prim. */

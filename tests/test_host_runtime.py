@@ -105,3 +105,59 @@ host.host_malloc_limit(1 << 40)
 assert lib.fx_ensemble_create(n, d, C.byref(h)) == 0
 lib.fx_ensemble_destroy(h)
 """)
+
+
+def test_transfers_where_staging_memory_is_short(host_run):
+    """A transfer that cannot have a larger staging buffer goes through the one
+    there is, in more chunks; where there is none, by 2D copies, which leave the
+    padding alone and bring the state back to the bit."""
+    host_run("""
+lib = _native.load()
+dp = C.POINTER(C.c_double)
+# 2D copies: no staging at all
+rng = np.random.default_rng(5)
+for mhd in (False, True):
+    n = (32, 16, 48)
+    m = GpuMesh(n, (0.0, 1.0) * 3, (0,) * 6, 1.4, mhd=mhd)
+    host.host_malloc_limit(0)
+    W = rng.standard_normal((m.nh,) + n)
+    bf = [rng.standard_normal([e + (a == d) for a, e in enumerate(n)]) for d in range(3)]
+    m.set_state(W, bf)
+    assert calls("hipMemcpy2DAsync") > 0
+    v = m.view()
+    for s in range(2):
+        assert np.array_equal(m.get_prim(s), W)
+        if mhd:
+            assert all(np.array_equal(a, b) for a, b in zip(m.get_bf(s), bf))
+        flat = np.ctypeslib.as_array(C.cast(v.W[s], dp), (m.nh, v.vstride)).copy()
+        i = (v.origin + np.arange(n[0])[:, None, None] * v.sx + np.arange(n[1])[:, None] * v.sy
+             + np.arange(n[2]))
+        assert np.array_equal(flat[:, i], W)
+        flat[:, i] = 0.0
+        assert not flat.any()
+    host.host_malloc_limit(1 << 40)
+    m.close()
+# a buffer that serves a small instance also serves a large one
+d = (_native.MeshDesc * 2)()
+for i in range(2):
+    d[i].n[:] = [16 + 48 * i] * 3
+    d[i].xlim[:] = [0.0, 1.0] * 3
+    d[i].gamma = 1.4
+h = C.c_void_p()
+_native.check(lib.fx_ensemble_create(2, d, C.byref(h)))
+W = [rng.standard_normal((6,) + (16 + 48 * i,) * 3) for i in range(2)]
+ptr = lambda a: a.ctypes.data_as(dp)
+_native.check(lib.fx_ensemble_set_prim(h, 0, ptr(W[0])))
+before = calls("hipMemcpy2DAsync"), calls("hipFree")
+host.host_malloc_limit(1 << 20)
+moved = calls("hipMemcpyAsync")
+_native.check(lib.fx_ensemble_set_prim(h, 1, ptr(W[1])))
+assert calls("hipMemcpyAsync") - moved == 1 + 64      # the time's reset, and 12.6 MB by 197 kB
+_native.check(lib.fx_ensemble_get_prim(h, 1, 0, ptr(W[1])))
+_native.check(lib.fx_ensemble_set_prim(h, 0, ptr(W[0])))
+assert (calls("hipMemcpy2DAsync"), calls("hipFree")) == before
+host.host_malloc_limit(1 << 40)
+_native.check(lib.fx_ensemble_set_prim(h, 1, ptr(W[1])))
+assert calls("hipFree") == before[1] + 1              # replaced by the larger one
+lib.fx_ensemble_destroy(h)
+""")

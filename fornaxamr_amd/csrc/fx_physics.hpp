@@ -444,8 +444,7 @@ __device__ __forceinline__ int hlld_outer(const HlldSide& s, double bx, double S
     double smdiff = S - SM;
     const bool coincide = fabs(smdiff) <= 1.0e-14 * (fabs(S) + fabs(SM) + 1.0);
     st.rho = s.rho * alpha / smdiff;
-    if (coincide | (st.rho <= 0.0) | !isfinite(st.rho))
-        return coincide ? HLLD_COINCIDE : HLLD_BAD_STAR_RHO;
+    const bool bad = coincide | (st.rho <= 0.0) | !isfinite(st.rho);
     st.vx = SM;
     st.ye = s.ye;
     double denom = s.rho * alpha * smdiff - bx * bx;
@@ -465,14 +464,14 @@ __device__ __forceinline__ int hlld_outer(const HlldSide& s, double bx, double S
     double vdotb = s.vx * bx + s.vy * s.by + s.vz * s.bz;
     double vsdotbs = st.vx * bx + st.vy * st.by + st.vz * st.bz;
     st.e = (alpha * s.e - s.pt * s.vx + pt_star * SM + bx * (vdotb - vsdotbs)) / smdiff;
-    return HLLD_OK;
+    return bad ? (coincide ? HLLD_COINCIDE : HLLD_BAD_STAR_RHO) : HLLD_OK;
 }
 
 // HLLD flux (src/prj_riemann.c:321-440).  WL/WR are rotated face states with
 // the normal field slot already set to bn.  Outputs the 9-variable flux, the
 // face velocity and the face EMFs Bv1 = bz*vx - bx*vz, Bv2 = bx*vy - by*vx of
 // the selected fan state (src/prj_riemann.c:305-319).  On an error the outputs
-// mean nothing.
+// mean nothing, but every one of them is set.
 //
 // Bound by instruction issue: a return behind each of the reference's dozen
 // checks cut the solver into as many masked regions, between which nothing is
@@ -489,6 +488,11 @@ __device__ __forceinline__ int hlld(const double* WL, const double* WR, double p
 {
     HlldSide L, R;
     int rc;
+    const auto refused = [&](int code) {
+        for (int v = 0; v < 9; ++v) flux[v] = 0.0;
+        vface[0] = vface[1] = vface[2] = *bv1 = *bv2 = 0.0;
+        return code;
+    };
     hlld_side(WL, pL, gL, bn, L);
     hlld_side(WR, pR, gR, bn, R);
     bool bad[4];
@@ -508,11 +512,12 @@ __device__ __forceinline__ int hlld(const double* WL, const double* WR, double p
                      (R.p <= 0.0) | (R.g <= 0.0) | bad[0] | bad[1] | bad[2] | bad[3] |
                      !(SL < SR);
     if (any) {
-        if ((rc = hlld_side_error(L)) != 0) return rc;
-        if ((rc = hlld_side_error(R)) != 0) return rc;
-        for (int c = 0; c < 4; ++c)
-            if (bad[c]) return c & 1 ? HLLD_BAD_CF : HLLD_BAD_DISC;
-        return HLLD_BAD_ORDER;
+        rc = HLLD_BAD_ORDER;
+        for (int c = 3; c >= 0; --c)
+            if (bad[c]) rc = c & 1 ? HLLD_BAD_CF : HLLD_BAD_DISC;
+        if (const int e = hlld_side_error(R)) rc = e;
+        if (const int e = hlld_side_error(L)) rc = e;
+        return refused(rc);
     }
 
     const bool sup_l = 0.0 <= SL;
@@ -520,7 +525,7 @@ __device__ __forceinline__ int hlld(const double* WL, const double* WR, double p
     double denom = R.rho * (SR - R.vx) - L.rho * (SL - L.vx);
     if (!sup && fabs(denom) <= 1.0e-14 * (fabs(R.rho * (SR - R.vx)) +
                                           fabs(L.rho * (SL - L.vx)) + 1.0))
-        return HLLD_BAD_CONTACT;
+        return refused(HLLD_BAD_CONTACT);
     double SM = (R.rho * R.vx * (SR - R.vx) - L.rho * L.vx * (SL - L.vx) + (L.pt - R.pt)) / denom;
     double ptl = L.pt + L.rho * (SL - L.vx) * (SM - L.vx);
     double ptr = R.pt + R.rho * (SR - R.vx) * (SM - R.vx);

@@ -46,27 +46,45 @@ constexpr int NT = 256;
 
 // Quotients by one divisor: its reciprocal by two Newton-Raphson steps from the
 // hardware's estimate, and per quotient the residual correction of Markstein
-// (IBM J. Res. Dev. 34, 1990): the bits of a / b wherever a and a / b are normal
-// numbers with 100 bits of exponent to spare below.  The divisor's exponent is
-// taken apart first, so no divisor over- or underflows on the way; the fixup
+// (IBM J. Res. Dev. 34, 1990).  The divisor is scaled into [1, 2) first, so that
+// nothing over- or underflows on the way that does not in the quotient; the fixup
 // gives zeros, infinities and NaN as the division does.  7 + 5 instructions per
-// quotient for 11 per division.
+// quotient for 11 per division (40 steps and their reverse at 64^3 8.41 ms, by
+// divisions 8.75; unguarded 8.33).
+//
+// The quotients are those of the division, to the bit, where every numerator is 0
+// or at least 2^-961 (its residual is then a number) and every quotient is normal.
+// exact() is whether that holds for all quotients formed so far in all lanes of
+// the wave; where it does not, the forward kernels form them again by division
+// (SHORT false), so that they round exactly whatever the state.  The reverse
+// kernels, which round as they like (hlle_vjp multiplies by a reciprocal), do not
+// ask: a quotient below that is off by a few units of the last place, or of the
+// smallest subnormal where the numerator is one.
+template <bool SHORT = true>
 struct Recip {
     double b, m, y;
     int e;
+    int least = 0;           // smallest exponent of a numerator (frexp's)
     __device__ __forceinline__ explicit Recip(double x) : b(x)
     {
-        m = __builtin_amdgcn_frexp_mant(x);
-        e = -__builtin_amdgcn_frexp_exp(x);
+        if (!SHORT) return;
+        e = 1 - __builtin_amdgcn_frexp_exp(x);
+        m = ldexp(x, e);
         y = __builtin_amdgcn_rcp(m);
         y = fma(y, fma(-m, y, 1.0), y);
         y = fma(y, fma(-m, y, 1.0), y);
     }
-    __device__ __forceinline__ double operator()(double a) const
+    __device__ __forceinline__ double operator()(double a)
     {
+        if (!SHORT) return a / b;
+        least = min(least, __builtin_amdgcn_frexp_exp(a));
         double q = a * y;
         q = fma(fma(-m, q, a), y, q);
         return __builtin_amdgcn_div_fixup(ldexp(q, e), b, a);
+    }
+    __device__ __forceinline__ bool exact() const
+    {
+        return !SHORT || __builtin_amdgcn_ballot_w64(least < max(-960, -1019 - e)) == 0;
     }
 };
 
@@ -88,7 +106,7 @@ __device__ __forceinline__ double va_d(double sl, double sr, double e, double& d
 {
     const double sl2 = sl * sl, sr2 = sr * sr;
     const double num = sl * (sr2 + e) + sr * (sl2 + e);
-    const Recip den((sl2 + sr2) + 2.0 * e);
+    Recip<> den((sl2 + sr2) + 2.0 * e);
     const double v = den(num);
     const double two_lr = 2.0 * sl * sr;
     dl = den((sr2 + e) + two_lr - v * (2.0 * sl));
@@ -108,7 +126,8 @@ struct HlleState {
     double U[6], F[6];
 };
 
-__device__ __forceinline__ void hlle_side(const double* a, const Recip& gm1, HlleState& s)
+template <typename Q>
+__device__ __forceinline__ void hlle_side(const double* a, Q& gm1, HlleState& s)
 {
     const double m = a[0] * a[1];
     const double ke = (0.5 * a[0]) * ((a[1] * a[1] + a[2] * a[2]) + a[3] * a[3]);
@@ -127,9 +146,10 @@ __device__ __forceinline__ void hlle_side(const double* a, const Recip& gm1, Hll
     s.F[5] = s.U[5] * a[1];
 }
 
-__device__ __forceinline__ void hlle(const double* qL, const double* qR, double gamma, double* F)
+template <bool SHORT>
+__device__ __forceinline__ bool hlle_by(const double* qL, const double* qR, double gamma, double* F)
 {
-    const Recip gm1(gamma - 1.0);
+    Recip<SHORT> gm1(gamma - 1.0);
     const double cL = sqrt((gamma * qL[4]) / qL[0]);
     const double cR = sqrt((gamma * qR[4]) / qR[0]);
     const double a1 = qL[1] - cL, a2 = qR[1] - cR;
@@ -142,12 +162,18 @@ __device__ __forceinline__ void hlle(const double* qL, const double* qR, double 
     hlle_side(qL, gm1, L);
     hlle_side(qR, gm1, R);
     const double bpm = bp * bm;
-    const Recip den(bp - bm);
+    Recip<SHORT> den(bp - bm);
 #pragma unroll
     for (int v = 0; v < 6; ++v) {
         const double num = (bp * L.F[v] - bm * R.F[v]) + bpm * (R.U[v] - L.U[v]);
         F[v] = den(num);
     }
+    return gm1.exact() && den.exact();
+}
+
+__device__ __forceinline__ void hlle(const double* qL, const double* qR, double gamma, double* F)
+{
+    if (!hlle_by<true>(qL, qR, gamma, F)) hlle_by<false>(qL, qR, gamma, F);
 }
 
 // weight of the first operand of min/max in the cotangent (1, 0 or 1/2 at a tie)
@@ -155,7 +181,7 @@ __device__ __forceinline__ double wfirst_min(double a, double b) { return a < b 
 __device__ __forceinline__ double wfirst_max(double a, double b) { return a > b ? 1.0 : (b > a ? 0.0 : 0.5); }
 
 // cotangent of one side's U and F back to its state a = (rho, u, v, w, p, Ye)
-__device__ __forceinline__ void hlle_side_vjp(const double* a, const Recip& gm1, const double* Ub,
+__device__ __forceinline__ void hlle_side_vjp(const double* a, Recip<>& gm1, const double* Ub,
                                               const double* Fb, double* ab)
 {
     const double rho = a[0], u = a[1], v = a[2], w = a[3], p = a[4], ye = a[5];
@@ -177,7 +203,7 @@ __device__ __forceinline__ void hlle_side_vjp(const double* a, const Recip& gm1,
 __device__ __forceinline__ void hlle_vjp(const double* qL, const double* qR, double gamma,
                                          const double* Fb, double* qLb, double* qRb)
 {
-    const Recip gm1(gamma - 1.0), rL(qL[0]), rR(qR[0]);
+    Recip<> gm1(gamma - 1.0), rL(qL[0]), rR(qR[0]);
     const double cL = sqrt(rL(gamma * qL[4]));
     const double cR = sqrt(rR(gamma * qR[4]));
     const double a1 = qL[1] - cL, a2 = qR[1] - cR;
@@ -351,9 +377,10 @@ __device__ __forceinline__ void cons6(const double* w, double* u)
     u[5] = w[0] * w[5];
 }
 
-__device__ __forceinline__ void prim6(const double* u, double* w)
+template <bool SHORT>
+__device__ __forceinline__ bool prim6(const double* u, double* w)
 {
-    const Recip r(u[0]);
+    Recip<SHORT> r(u[0]);
     w[0] = u[0];
     w[1] = r(u[1]);
     w[2] = r(u[2]);
@@ -361,6 +388,7 @@ __device__ __forceinline__ void prim6(const double* u, double* w)
     const double m2 = (u[1] * u[1] + u[2] * u[2]) + u[3] * u[3];
     w[4] = r(u[4] - r(0.5 * m2));
     w[5] = r(u[5]);
+    return r.exact();
 }
 
 // The z direction and the update of a forward stage.  Wave w of the launch has
@@ -405,7 +433,6 @@ __global__ void __launch_bounds__(NT, 4) adj_stage_kernel(AdjGeom g, double dt,
     for (int v = 0; v < 6; ++v)
         sum[v] = ((0.0 + g.area[0] * dF[v * N + c]) + g.area[1] * dF[(6 + v) * N + c]) +
                  g.area[2] * dz[v];
-    const Recip vol(g.vol);
 
     double wc[6], u[6], u0[6], u1[6], wn[6];
 #pragma unroll
@@ -417,13 +444,20 @@ __global__ void __launch_bounds__(NT, 4) adj_stage_kernel(AdjGeom g, double dt,
         for (int v = 0; v < 6; ++v) w0[v] = W0[v * N + c];
         cons6(w0, u0);
     }
+    double fd[6];
+    Recip<> vol(g.vol);
+#pragma unroll
+    for (int v = 0; v < 6; ++v) fd[v] = vol(0.0 - sum[v]);
+    if (!vol.exact()) {
+#pragma unroll
+        for (int v = 0; v < 6; ++v) fd[v] = (0.0 - sum[v]) / g.vol;
+    }
 #pragma unroll
     for (int v = 0; v < 6; ++v) {
-        const double fd = vol(0.0 - sum[v]);
-        const double ut = u[v] + dt * fd;
+        const double ut = u[v] + dt * fd[v];
         u1[v] = STAGE == 1 ? ut : 0.5 * u0[v] + 0.5 * ut;
     }
-    prim6(u1, wn);
+    if (!prim6<true>(u1, wn)) prim6<false>(u1, wn);
 #pragma unroll
     for (int v = 0; v < 6; ++v) Wout[v * N + c] = wn[v];
 }

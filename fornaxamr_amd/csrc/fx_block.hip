@@ -121,6 +121,7 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
     const int np = BS / split;
     const int x0 = (wg % split) * np;
     const int x1 = x0 + np == BS ? BS + 1 : x0 + np;   // the last part adds x-face 16
+    // faces x0 .. x1 - 1 need the cells of planes x0 - 2 .. x1
     const int64_t vs = bp->var_stride;
     const double* __restrict__ W = as_global(bp->W);
     const double* __restrict__ eos = as_global(bp->eosvar);
@@ -235,7 +236,7 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
         const double v3m = W[3 * vs + o + oidx - 1], v3p = W[3 * vs + o + oidx + 1];
         load_plane(x0, c0, h0);
         load_plane(x0 + 1, c1, h1);
-        load_plane(x0 + 2 <= BS + 1 ? x0 + 2 : BS + 1, own, halo);
+        if (x0 + 2 <= x1) load_plane(x0 + 2, own, halo);
         dy = dmin_delta(cm.q[2] - v2m, v2p - cm.q[2]);
         dz = dmin_delta(cm.q[3] - v3m, v3p - cm.q[3]);
 #pragma unroll
@@ -352,16 +353,12 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
         }
         if (i + 1 == x1) break;
         // ---- plane i + 2 -------------------------------------------------------------
-        if (i + 2 <= BS + 1) {
-            L.v1[(n + 2) & 3][oidx] = own.q[1];
-            if (has_halo) L.v1[(n + 2) & 3][hidx] = halo.q[1];
-        }
+        L.v1[(n + 2) & 3][oidx] = own.q[1];
+        if (has_halo) L.v1[(n + 2) & 3][hidx] = halo.q[1];
         __syncthreads();
-        if (i + 2 <= BS + 1) {
-            store_cell(A, oidx, own);
-            if (has_halo) store_cell(A, hidx, halo);
-        }
-        if (i + 3 <= BS + 1) load_plane(i + 3, own, halo);
+        store_cell(A, oidx, own);
+        if (has_halo) store_cell(A, hidx, halo);
+        if (i + 3 <= x1) load_plane(i + 3, own, halo);
     }
 }
 

@@ -369,8 +369,8 @@ def main():
                     "default 256 (hydro), 128 (mhd)")
     ap.add_argument("--mhd-schedule", default=None, metavar="CT,SIDE",
                     help="MHD launch schedule instead of the automatic one: CT workgroups "
-                         "per block (1, 2, 4) and the ghost-layer faces in order (0) or on "
-                         "a second stream (1), e.g. 1,0 (fx_mesh_set_mhd_schedule)")
+                         "per block (1, 2, 4; 0 automatic) and SIDE (0, 1 or -1), which changes "
+                         "nothing any more, e.g. 1,0 (fx_mesh_set_mhd_schedule)")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline")
     ap.add_argument("--no-ensemble", action="store_true", help="skip the batched-ensemble figure")
     ap.add_argument("--no-mhd", action="store_true",

@@ -16,7 +16,7 @@
 // overlaps.  A stage is two launches: the x and y directions, then the z direction
 // and the sum at each cell.  Bound: half by the FP64 instructions, half by the
 // 113 MB (forward) and 155 MB (reverse) that a 64^3 stage moves, at 5 TB/s.
-// us at 64^3: forward stage 15.8 + 13.5, reverse stage 29.4 + 22.5; a face kernel
+// us at 64^3: forward stage 15.4 + 12.5, reverse stage 28.1 + 21.5; a face kernel
 // and a cell kernel, all face values or cotangents through memory and each slope
 // formed by every face that uses it, took 22 + 11 and 33 + 43.  One forward launch
 // in which a lane formed both its x- and y-faces took 34 (2711 instructions a

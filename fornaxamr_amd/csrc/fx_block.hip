@@ -368,7 +368,7 @@ __global__ void __launch_bounds__(NT, 2) block_march_kernel(const fx_block_io* _
 // 1024 lanes solve a face.  Four whole planes (i - 2 .. i + 1, 11 quantities,
 // 140,800 B) are in LDS, so that a face of any direction is one stencil of four
 // cells and the HLLD code appears once; thread t < 400 holds cell t of the next
-// plane in registers meanwhile.  One workgroup per CU, two waves per SIMD, 48 %
+// plane in registers meanwhile.  One workgroup per CU, two waves per SIMD, 46-53 %
 // VALU issue; sixteen waves of one task each (128 VGPRs) spilled 128 and took
 // 421 us where this takes 291 (256 blocks).
 //
@@ -583,6 +583,11 @@ hipError_t launch_block_flux(const fx_block_io* blocks_dev, int n, int mhd, int*
         const int nwg = (int)std::min<int64_t>((int64_t)n * MP, std::max(ncu, 1));
         hipLaunchKernelGGL(block_march_mhd_kernel, dim3(nwg), dim3(NTM), 0, s, blocks_dev, n, err);
     } else {
+        // The rule of the mesh stage, whose constants are not this kernel's (its stores
+        // outlast a prologue): of all five splits on 21 counts from 1 to 4096 blocks its
+        // choice was the fastest, or within 5 % of it, but for 400 blocks (268 us at
+        // split 2; whole 249, split 8 240).  1 block 101 -> 12 us (16), 64 103 -> 30 (8),
+        // 128 104 -> 61 (4), 256 154 -> 148 (2); 1000 and 4096 stay whole.
         const int split = stage_split(n, ncu);
         hipLaunchKernelGGL(block_march_kernel, dim3(n * split), dim3(NT), 0, s, blocks_dev, split);
     }

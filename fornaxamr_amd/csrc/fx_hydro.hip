@@ -692,8 +692,9 @@ __global__ void queue_reset_kernel(int* q)
 }  // namespace
 
 // Shared with the MHD flux kernel, which marches the same way at the same two
-// workgroups per CU.  A workgroup of np planes costs a prologue (the stencil's
-// planes, an extra x-face) and np plane steps; 2 ncu workgroups run at once.  In plane steps: one round
+// workgroups per CU, with the batched ensemble stages and with the per-block hydro
+// kernel.  A workgroup of np planes costs a prologue (the stencil's planes, an extra
+// x-face) and np plane steps; 2 ncu workgroups run at once.  In plane steps: one round
 // costs 1.5 + np (0.8 of it where every CU holds one workgroup at most), and in
 // longer runs, where prologues overlap other workgroups' planes, each full
 // round 0.85 + np and the last one 0.68 or 0.97 of that.  The constants are
@@ -704,7 +705,9 @@ __global__ void queue_reset_kernel(int* q)
 // 114 -> 48 us (4), 216 blocks 113 -> 78 us (2), 343 blocks 148 -> 122 us (4);
 // 512 blocks stay whole (141 us, split 2: 146), as do 4096.  MHD step by the
 // flux split alone: 8 blocks 597 -> 158 us (16), 64 blocks 616 -> 249 us (8),
-// 125 blocks 648 -> 354 us (4), 216 blocks 715 -> 553 us (2).
+// 125 blocks 648 -> 354 us (4), 216 blocks 715 -> 553 us (2).  Batched ensemble steps
+// of 16 to 1728 blocks, 13 mixes: within 1.5 % of the fastest split (16 blocks 213 -> 32
+// us, 120: 227 -> 96, 288: 275 -> 219, 768: 491 -> 427 where split 2 takes 423).
 int stage_split(int64_t nblocks, int ncu)
 {
     int best = 1;

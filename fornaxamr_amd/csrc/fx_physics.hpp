@@ -478,8 +478,8 @@ __device__ __forceinline__ int hlld_outer(const HlldSide& s, double bx, double S
 // scheduled.  One branch holds the checks of both states, and the supersonic, single-
 // and double-star fluxes are stages of one sum rather than separate exits.
 // MHD step: 256^3 7.54 -> 6.87 ms, 128^3 1041 -> 957 us, 48x32x64 120 -> 114.
-// SHORT: with the short forms of the fast speeds (256^3 7.00 -> 6.88 ms per step,
-// 112x48x80 274 -> 268 us; not worth it in the per-block kernel, whose one
+// SHORT: with the short forms of the fast speeds (256^3 7.00 -> 6.88 ms per step on a
+// slower card, 112x48x80 274 -> 268 us; not worth it in the per-block kernel, whose one
 // workgroup per CU of 8 waves gains nothing: 343 blocks 390 -> 392 us).
 template <bool SHORT = true>
 __device__ __forceinline__ int hlld(const double* WL, const double* WR, double pL, double pR,

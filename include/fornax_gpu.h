@@ -99,12 +99,6 @@ int fx_step_dt(fx_mesh *m, double dt);
 #define FX_RK2 0
 #define FX_ESSPRK10_4 1
 int fx_mesh_set_integrator(fx_mesh *m, int integrator);
-/* Riemann solver of a hydro mesh's stage.  FX_RIEMANN_HLLC (default): the
- * reference's prj_riemann_hllc with the theta limiter (src/prj_riemann.c:
- * 1494-1599).  FX_RIEMANN_HLLE: HLL over the same Davis wave-speed bounds and
- * face states, in the form of the reference's HLL fallback
- * (src/prj_riemann.c:393-407); the reference has no hydro HLLE, so this
- * option has no reference counterpart.  MHD meshes take HLLD only. */
 /* Launch schedule of an MHD mesh's stage (no reference counterpart; every
  * schedule gives the same bits).  ct_split: CT workgroups per block, 1, 2 or
  * 4 (each marches 16/ct_split of the block's x-planes), 0 automatic (up to 16
@@ -112,6 +106,12 @@ int fx_mesh_set_integrator(fx_mesh *m, int integrator);
  * -1; the ghost-layer faces run in the flux kernel's launch whichever is given
  * (1 once meant a second stream).  Synchronises the mesh's stream first. */
 int fx_mesh_set_mhd_schedule(fx_mesh *m, int ct_split, int side_stream);
+/* Riemann solver of a hydro mesh's stage.  FX_RIEMANN_HLLC (default): the
+ * reference's prj_riemann_hllc with the theta limiter (src/prj_riemann.c:
+ * 1494-1599).  FX_RIEMANN_HLLE: HLL over the same Davis wave-speed bounds and
+ * face states, in the form of the reference's HLL fallback
+ * (src/prj_riemann.c:393-407); the reference has no hydro HLLE, so this
+ * option has no reference counterpart.  MHD meshes take HLLD only. */
 #define FX_RIEMANN_HLLC 0
 #define FX_RIEMANN_HLLE 1
 int fx_mesh_set_riemann(fx_mesh *m, int solver);
